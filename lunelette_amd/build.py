@@ -124,7 +124,7 @@ def build_library(jobs=8):
 def build_oracle():
     _run(["make", "-s", "-C", os.path.join(ROOT, "oracle")])
     ref = "/root/reference"
-    if os.path.isdir(ref):
+    if os.path.isfile(os.path.join(ref, "src", "safetensors.c")):
         _run(["make", "-s", "-C", os.path.join(ROOT, "oracle"), "-f", "Makefile.ref",
               "REF=" + ref])
 
