@@ -21,6 +21,20 @@ int lh_launch_qkv_rope(int lookup, const uint8_t *Wqkv, float sq, float sk, floa
     float *q, float *kcache_layer, float *vcache_layer, uint32_t capacity, hipStream_t s);
 int lh_launch_gateup_silu(int lookup, const uint8_t *Wgate, const uint8_t *Wup, float sg,
     float su, const float *gamma, const float *x, uint32_t count, float *gated, hipStream_t s);
+/* Multi-token projections on the FP32 matrix instructions (precise.hip); xt:
+ * activations in tile order, whole 16-token tiles (rows past count are read,
+ * never used). resident: FP32 weights, otherwise FP8 codes. */
+int lh_launch_norm_tile(const float *x, const float *gamma, float *xt, uint32_t count,
+    hipStream_t s);
+int lh_launch_tile_rows(const float *x, float *xt, uint32_t count, hipStream_t s);
+int lh_launch_qkv_tile(int resident, const void *Wqkv, float sq, float sk, float sv,
+    const float *xt, const lh_step_params *params, uint32_t count, float *q, float *kcache_layer,
+    float *vcache_layer, uint32_t capacity, hipStream_t s);
+int lh_launch_gateup_tile(int resident, const void *Wgate, const void *Wup, float sg, float su,
+    const float *xt, uint32_t count, float *gated_xt, hipStream_t s);
+/* x += scale * rows of the 3072 x cols projection (cols 4096 or 9216). */
+int lh_launch_residual_tile(int resident, const void *W, float scale, uint32_t cols,
+    const float *xt, uint32_t count, float *x, hipStream_t s);
 /* nonfinite (may be NULL) is set to 1 when any written logit is Inf or NaN. */
 int lh_launch_head(const uint16_t *E, const float *gamma, const float *xrow, float *logits,
     uint32_t *nonfinite, hipStream_t s);

@@ -1,0 +1,504 @@
+// Projections of the precise multi-token path (prefill mode CUSTOM and every
+// multi-token call of the resident strategy) on the FP32 matrix
+// instructions, bit for bit the canonical row dots of the decode kernels
+// (lh_schedule.h).
+//
+// v_mfma_f32_16x16x1_4b_f32 is four independent 16 x 16 outer products whose
+// every element is one correctly rounded fused multiply-add (subnormals kept),
+// so a run of them is exactly the canonical chain acc = fma(w, x, acc): block
+// b of an instruction holds one lane-chain of the schedule for 16 tokens x 16
+// weight rows. The 64 chains of a dot are split over the workgroup's eight
+// waves by chain number mod 8: wave s owns chains 8m + s, m = 4g + b, as two
+// accumulators g of four blocks b each, so the first three levels of the
+// halving tree (distances 32, 16, 8) add inside the wave's registers and the
+// last three (4, 2, 1) join the eight waves through LDS.
+//
+// Activations arrive in the tile order of lh_xt_word (written by the producing
+// kernel): a wave's operand for one (chunk, g) is four contiguous 1 KiB loads
+// straight to registers, since no other wave of the workgroup reads it. Weight
+// rows stay as stored; one stage (16 RT rows x 512 columns, every wave's
+// chains of one g) goes to LDS by direct loads of whole row segments, its
+// 16-byte words XOR-permuted by row so that the operand reads (16 rows, one
+// column word each) are free of bank conflicts. FP8 codes decode in registers
+// (v_cvt_pk_f32_fp8, exact). The next stages' loads are in flight while this
+// one's 16 RT MFMAs per wave run.
+//
+// Bound: the FP32 matrix rate (32 products per SIMD and cycle; 59.6 GFLOP of a
+// layer's projections at 256 tokens take 0.45 ms at the 2.0 GHz the chip
+// holds under this load). Measured there 0.61 ms (65 to 75% of that rate),
+// where the row dots it replaces, one token per workgroup, took 3.7 ms (each
+// token read and decoded every weight again: 16 TFLOP/s).
+#include "lh_device.h"
+#include "lh_internal.h"
+
+namespace lh {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+enum { K_FP8 = 0, K_F32 = 2 };
+enum { EPI_RESIDUAL, EPI_QKV, EPI_GATEUP };
+
+struct TileArgs {
+    const char* W;         // weight rows (q|k|v, o, gate, down)
+    const char* W1;        // up rows (EPI_GATEUP)
+    float s0, s1, s2;      // tensor scales (q, k, v; gate, up; or the one scale)
+    const f32x4* xt;       // activations, lh_xt_word order
+    uint32_t count;        // tokens
+    uint32_t tiles;        // row tiles * token tiles
+    uint32_t token_tiles;  // ceil(count / 16)
+    float* x;              // EPI_RESIDUAL: rows of 3072, updated in place
+    const lh_step_params* params;  // EPI_QKV
+    float* q;
+    float* kcache;
+    float* vcache;
+    uint32_t capacity;
+    f32x4* gated;          // EPI_GATEUP: lh_xt_word order, 9216 columns
+};
+
+// 16-byte word of (token t, columns col .. col + 3) in the activation tile
+// order of a K-column projection; col % 4 == 0. Tiles of 16 tokens; in a tile
+// [chunk][g][wave s][quad][block b][token % 16], col = 1024 chunk + 512 g +
+// 128 b + 16 s + 4 quad.
+__device__ __forceinline__ size_t lh_xt_word(uint32_t t, uint32_t col, uint32_t K)
+{
+    const uint32_t cg = col >> 9, b = (col >> 7) & 3, sq = (col >> 2) & 31;
+    return ((size_t)(t >> 4) * (K >> 9) + cg) * 2048 + sq * 64 + b * 16 + (t & 15);
+}
+
+// The weight rows of a workgroup's 16 RT tile rows n. EPI_RESIDUAL: consecutive
+// rows. EPI_QKV: the lower halves of 8 RT consecutive RoPE pairs of one head,
+// then their upper halves. EPI_GATEUP: 8 RT gate rows, then the matching up
+// rows (of W1). tile_base: the first row; tile_row: row n relative to it, the
+// same for every tile.
+template <int RT, int EPI>
+__device__ __forceinline__ uint32_t tile_base(uint32_t rt)
+{
+    constexpr uint32_t NP = 8 * RT;
+    return EPI == EPI_RESIDUAL ? rt * 16 * RT
+        : EPI == EPI_QKV ? (rt * NP >> 6) * 128 + (rt * NP & 63) : rt * NP;
+}
+
+template <int RT, int EPI>
+__device__ __forceinline__ uint32_t tile_row(uint32_t n)
+{
+    constexpr uint32_t NP = 8 * RT;
+    return EPI == EPI_RESIDUAL || n < NP ? n : n - NP + (EPI == EPI_QKV ? 64 : 0);
+}
+
+// Tiles of 16 tokens x 16 RT weight rows of a K = 1024 NCH projection.
+// Workgroup id (512 threads) takes tiles id, id + gridDim.x, ...; gridDim.x and the
+// row tiles are multiples of 8. Tile j's token tiles follow each other on XCD
+// j % 8, so a row tile's weights come from HBM once. A tile's first stage is
+// requested during the last stages of the tile before it and lands under that
+// tile's reduction and epilogue.
+template <int KIND, int NCH, int RT, int EPI>
+__device__ __forceinline__ void tile_body(const TileArgs& a)
+{
+    constexpr uint32_t K = NCH * LH_CHUNK, ES = KIND == K_FP8 ? 1 : 4;
+    constexpr uint32_t ROW_WORDS = 512 * ES / 16;       // LDS words of a row's stage
+    constexpr uint32_t STAGE_WORDS = 16 * RT * ROW_WORDS;
+    constexpr int LOADS = STAGE_WORDS / 512;            // direct loads per wave and stage
+    constexpr int WQ = ES;                              // LDS words per lane and (row, chain)
+    constexpr uint32_t NP = 8 * RT;
+    constexpr uint32_t RS = 16 * RT + 4;                // reduction row stride: no bank conflicts
+    // The 2 NCH stages of a tile take NB buffers in turn, a whole number of
+    // turns per tile, NB - 1 stages of weights ahead; FP32 rows and the
+    // 8-stage projection keep to two, so that two workgroups fit a CU's LDS.
+    constexpr int STAGES = 2 * NCH, NB = STAGES % 3 || KIND == K_F32 ? 2 : 3;
+    constexpr int UNROLL = 2 * (NB == 3 ? 3 : 1), AHEAD = NB - 1;
+    __shared__ u32x4 w0[STAGE_WORDS];
+    __shared__ u32x4 w1[STAGE_WORDS];
+    __shared__ u32x4 w2[NB == 3 ? STAGE_WORDS : 1];
+    __shared__ __attribute__((aligned(16))) float red[8 * 16 * RS];
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t s = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t tile = blockIdx.x, tt, rt;
+    // Scalar offsets of the stage loads (the tensors are below 4 GiB).
+    const char* const W = EPI == EPI_GATEUP && s >= 4 ? a.W1 : a.W;
+    uint32_t src, xsrc;
+    // Direct loads: load i of wave s fills LDS words (s * LOADS + i) * 64 + lane,
+    // row n = word / ROW_WORDS; LDS word w of row n holds the row's word w ^ (n & 15).
+    // Waves 0..3 load the lower half of the rows.
+    uint32_t off[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) {
+        const uint32_t word = (s * LOADS + i) * 64 + lane;
+        const uint32_t n = word / ROW_WORDS, w = word % ROW_WORDS;
+        off[i] = tile_row<RT, EPI>(n) * K * ES + 16 * (w ^ (n & 15));
+    }
+    auto locate = [&](uint32_t j) {
+        const uint32_t rest = j >> 3;
+        tt = rest % a.token_tiles;
+        rt = (rest / a.token_tiles) * 8 + (j & 7);
+    };
+    auto weights = [&]() { src = tile_base<RT, EPI>(rt) * K * ES; };
+    auto activations = [&]() { xsrc = (tt * (K >> 9) * 2048 + s * 256) * 16; };
+    auto load_w = [&](uint32_t stage, u32x4* buf) {
+        const char* p = W + __builtin_amdgcn_readfirstlane(src + stage * 512 * ES);
+#pragma unroll
+        for (int i = 0; i < LOADS; i++) {
+            __builtin_amdgcn_global_load_lds(p + off[i], buf + (s * LOADS + i) * 64, 16, 0, 0);
+        }
+    };
+    f32x4 xn[4], xc[4];
+    auto load_x = [&](uint32_t stage) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(a.xt) +
+            __builtin_amdgcn_readfirstlane(xsrc + stage * 2048 * 16));
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            xn[i] = p[i * 64 + lane];
+        }
+    };
+    // Operand words of row tile r: row n = 16 r + lane % 16, chain 8 (lane / 16) + s.
+    const uint32_t n16 = lane & 15, wbase = ((lane >> 4) * 8 + s) * WQ;
+    f32x16 acc[RT][2];
+    auto compute = [&](const u32x4* buf, int g) {
+        u32x4 raw[RT][KIND == K_FP8 ? 1 : 4];
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+#pragma unroll
+            for (int i = 0; i < WQ; i++) {
+                raw[r][i] = buf[(16 * r + n16) * ROW_WORDS + ((wbase + i) ^ n16)];
+            }
+        }
+        // Columns 4i .. 4i + 3 of the chains, decoded while the four columns
+        // before them multiply. The scheduling barriers let only vector and
+        // scalar arithmetic cross, so consecutive MFMAs belong to different
+        // row tiles and the stage's loads stay where they are issued.
+        float w[2][RT][4];
+        auto decode = [&](int i) {
+#pragma unroll
+            for (int r = 0; r < RT; r++) {
+                if constexpr (KIND == K_FP8) {
+                    fp8x4_to_f32(raw[r][0][i], w[i & 1][r]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        w[i & 1][r][e] = __uint_as_float(raw[r][i][e]);
+                    }
+                }
+            }
+        };
+        decode(0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (i < 3) {
+                decode(i + 1);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+#pragma unroll
+                for (int r = 0; r < RT; r++) {
+                    acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x1f32(xc[i][e], w[i & 1][r][e],
+                        acc[r][g], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0x6);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Four rows n .. n + 3 of token t of the tile: levels 4, 2 and 1 over the waves.
+    auto total4 = [&](uint32_t t, uint32_t n) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(red + t * RS + n);
+        f32x4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            v[i] = p[i * 16 * RS / 4];
+        }
+        return ((v[0] + v[4]) + (v[2] + v[6])) + ((v[1] + v[5]) + (v[3] + v[7]));
+    };
+    if (tile >= a.tiles) {
+        return;
+    }
+    locate(tile);
+    weights();
+    activations();
+    load_w(0, w0);
+    load_x(0);
+    if (AHEAD == 2) {
+        load_w(1, w1);
+    }
+    u32x4* const bufs[3] = {w0, w1, w2};
+    while (true) {
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            acc[r][0] = acc[r][1] = f32x16{};
+        }
+        const uint32_t t0 = tt * 16, n0 = rt;
+        const bool more = tile + gridDim.x < a.tiles;
+        for (int st = 0; st < STAGES; st += UNROLL) {
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) {
+                const int k = st + u;
+                // Stage k has landed in every wave's part (two ahead, stage
+                // k + 1's weight loads, issued last, may be in flight), and
+                // every wave has read the buffer of stage k - 1.
+                __builtin_amdgcn_s_waitcnt(0x0f70 | (AHEAD == 2 ? LOADS : 0));
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    xc[i] = xn[i];
+                }
+                // Stage k + 1's activations, then stage k + AHEAD's weights;
+                // past this tile's last stage, the next tile's (the last
+                // tile requests its own first stages again, unused).
+                if (k + AHEAD == STAGES) {
+                    tile = more ? tile + gridDim.x : tile;
+                    locate(tile);
+                    weights();
+                }
+                if (k + 1 == STAGES) {
+                    activations();
+                }
+                load_x(k + 1 < STAGES ? k + 1 : 0);
+                load_w(k + AHEAD < STAGES ? k + AHEAD : k + AHEAD - STAGES,
+                    bufs[(u + AHEAD) % NB]);
+                __builtin_amdgcn_sched_barrier(0);
+                compute(bufs[u % NB], u & 1);
+            }
+        }
+        // Tree levels 32 (the two accumulators), 16 and 8 (their blocks): lane
+        // holds tokens 4 (lane / 16) + k, row lane % 16 of each row tile.
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            const f32x16 v = acc[r][0] + acc[r][1];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                red[(s * 16 + 4 * (lane >> 4) + k) * RS + 16 * r + n16] =
+                    (v[k] + v[8 + k]) + (v[4 + k] + v[12 + k]);
+            }
+        }
+        // LDS only: the next tile's first stage stays in flight.
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if constexpr (EPI == EPI_RESIDUAL) {
+            const uint32_t tl = tid / (4 * RT), n = tid % (4 * RT) * 4, t = t0 + tl;
+            if (tid < 64 * RT && t < a.count) {
+                f32x4* px = reinterpret_cast<f32x4*>(a.x + (size_t)t * LH_HIDDEN +
+                    n0 * 16 * RT + n);
+                const f32x4 old = *px, v = total4(tl, n);
+                *px = old + v * a.s0;
+            }
+        } else if constexpr (EPI == EPI_QKV) {
+            const uint32_t tl = tid / (2 * RT), n = tid % (2 * RT) * 4, t = t0 + tl;
+            if (tid < 32 * RT && t < a.count) {
+                const uint32_t pair = n0 * NP + n, head = pair >> 6, i = pair & 63;
+                const float scale = head < 32 ? a.s0 : (head < 40 ? a.s1 : a.s2);
+                const f32x4 lo = total4(tl, n) * scale, hi = total4(tl, n + NP) * scale;
+                const lh_token_params* tp = &a.params->tokens[t];
+                const uint32_t position = a.params->length + t;
+                if (head < 40) {
+                    // column i < 64 rotates with -x[i+64]; column i+64 with x[i].
+                    const f32x4 cl = *reinterpret_cast<const f32x4*>(tp->cosine + i);
+                    const f32x4 sl = *reinterpret_cast<const f32x4*>(tp->sine + i);
+                    const f32x4 ch = *reinterpret_cast<const f32x4*>(tp->cosine + i + 64);
+                    const f32x4 sh = *reinterpret_cast<const f32x4*>(tp->sine + i + 64);
+                    f32x4 out_lo = lo * cl + (-hi) * sl;
+                    f32x4 out_hi = hi * ch + lo * sh;
+                    if (head < 32) {
+                        f32x4* qh = reinterpret_cast<f32x4*>(a.q + (size_t)t * LH_QUERY +
+                            head * 128 + i);
+                        qh[0] = out_lo * tp->qfactor;
+                        qh[16] = out_hi * tp->qfactor;
+                    } else {
+                        *reinterpret_cast<f32x4*>(a.kcache +
+                            lh_k_index(a.capacity, 0, head - 32, position, i)) = out_lo;
+                        *reinterpret_cast<f32x4*>(a.kcache +
+                            lh_k_index(a.capacity, 0, head - 32, position, i + 64)) = out_hi;
+                    }
+                } else {
+                    f32x4* vr = reinterpret_cast<f32x4*>(a.vcache +
+                        lh_kv_index(a.capacity, 0, head - 40, position) + i);
+                    vr[0] = lo;
+                    vr[16] = hi;
+                }
+            }
+        } else {
+            // One word of the next projection's tile order per thread. Rows
+            // past count are written too (their products are never stored).
+            const uint32_t tl = tid & 15, n = (tid >> 4) * 4;
+            if (tid < 32 * RT) {
+                const f32x4 g = total4(tl, n) * a.s0, u = total4(tl, n + NP) * a.s1;
+                f32x4 y;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    y[k] = silu(g[k]) * u[k];
+                }
+                a.gated[lh_xt_word(t0 + tl, n0 * NP + n, LH_INNER)] = y;
+            }
+        }
+        if (!more) {
+            // The unused direct loads land before the LDS is given back.
+            __builtin_amdgcn_s_waitcnt(0);
+            return;
+        }
+    }
+}
+
+// (The body is device code only: the host pass has no matrix instructions.)
+template <int KIND, int NCH, int RT, int EPI>
+__global__ void __launch_bounds__(512, 4)
+k_tile(TileArgs a)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    tile_body<KIND, NCH, RT, EPI>(a);
+#endif
+}
+
+// Canonical RMSNorm of a 3072-wide row per workgroup, written in the tile
+// order of the next projection. grid (count), block 768: thread i owns columns
+// 4i .. 4i+3.
+__global__ void __launch_bounds__(768)
+k_norm_tile(const float* __restrict__ x, const float* __restrict__ gamma, f32x4* __restrict__ xt)
+{
+    // Lane l's 16 values of chunk c (columns c*1024 + 16l .. +15) are words
+    // (4c + q)*64 + l.
+    __shared__ f32x4 row_l[LH_HIDDEN / 4];
+    __shared__ float r_s;
+    const uint32_t t = blockIdx.x, tid = threadIdx.x;
+    const f32x4 g = reinterpret_cast<const f32x4*>(gamma)[tid];
+    const f32x4 v = reinterpret_cast<const f32x4*>(x + (size_t)t * LH_HIDDEN)[tid];
+    const uint32_t c = tid >> 8, w = tid & 255;
+    row_l[(4 * c + (w & 3)) * 64 + (w >> 2)] = v;
+    __syncthreads();
+    if (tid < 64) {
+        float acc = 0.0f;
+#pragma unroll
+        for (int k = 0; k < LH_HIDDEN / 256; k++) {
+            const f32x4 u = row_l[k * 64 + tid];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                acc = __builtin_fmaf(u[e], u[e], acc);
+            }
+        }
+        const float ss = wave_tree64(acc);
+        if (tid == 0) {
+            r_s = 1.0f / __builtin_sqrtf(ss / (float)LH_HIDDEN + 1e-5f);
+        }
+    }
+    __syncthreads();
+    const float r = r_s;
+    f32x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        y[e] = g[e] * (v[e] * r);
+    }
+    xt[lh_xt_word(t, 4 * tid, LH_HIDDEN)] = y;
+}
+
+// Attention output rows of 4096 into the o projection's tile order. grid
+// (count), block 1024: thread i owns columns 4i .. 4i+3.
+__global__ void __launch_bounds__(1024)
+k_tile_rows(const f32x4* __restrict__ x, f32x4* __restrict__ xt)
+{
+    const uint32_t t = blockIdx.x, tid = threadIdx.x;
+    xt[lh_xt_word(t, 4 * tid, LH_QUERY)] = x[(size_t)t * (LH_QUERY / 4) + tid];
+}
+
+}  // namespace lh
+
+using namespace lh;
+
+static int launched()
+{
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// Two workgroups fit a CU (128 registers, at most 76 KB of LDS).
+template <int KIND, int NCH, int RT, int EPI>
+static void launch_tile(uint32_t rows, TileArgs a, hipStream_t s)
+{
+    a.tiles = rows / (16 * RT) * a.token_tiles;
+    hipLaunchKernelGGL((k_tile<KIND, NCH, RT, EPI>), dim3(a.tiles < 512 ? a.tiles : 512),
+        dim3(512), 0, s, a);
+}
+
+// FP8 projections take two row tiles per workgroup where that leaves no CU
+// with more of them than single ones would (the CU with the most work holds
+// ceil(workgroups / 256) workgroups): at 256 tokens 0.61 ms a layer against
+// 0.66 ms with one, at 16 tokens 77 against 62 us. Four per workgroup (one
+// resident per CU) measured the same as two at 256 tokens and worse below.
+// FP32 rows take one: their stages are four times as large.
+template <int KIND, int NCH, int EPI>
+static int run_tile(uint32_t rows, const TileArgs& a, hipStream_t s)
+{
+    const uint32_t single = rows / 16 * a.token_tiles;
+    if constexpr (KIND == K_FP8) {
+        if ((single / 2 + 255) / 256 * 2 <= (single + 255) / 256) {
+            launch_tile<KIND, NCH, 2, EPI>(rows, a, s);
+            return launched();
+        }
+    }
+    launch_tile<KIND, NCH, 1, EPI>(rows, a, s);
+    return launched();
+}
+
+extern "C" int lh_launch_norm_tile(const float* x, const float* gamma, float* xt, uint32_t count,
+    hipStream_t s)
+{
+    hipLaunchKernelGGL(k_norm_tile, dim3(count), dim3(768), 0, s, x, gamma,
+        reinterpret_cast<f32x4*>(xt));
+    return launched();
+}
+
+extern "C" int lh_launch_tile_rows(const float* x, float* xt, uint32_t count, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_tile_rows, dim3(count), dim3(1024), 0, s,
+        reinterpret_cast<const f32x4*>(x), reinterpret_cast<f32x4*>(xt));
+    return launched();
+}
+
+extern "C" int lh_launch_qkv_tile(int resident, const void* Wqkv, float sq, float sk, float sv,
+    const float* xt, const lh_step_params* params, uint32_t count, float* q, float* kcache_layer,
+    float* vcache_layer, uint32_t capacity, hipStream_t s)
+{
+    TileArgs a = {};
+    a.W = static_cast<const char*>(Wqkv);
+    a.s0 = sq, a.s1 = sk, a.s2 = sv;
+    a.xt = reinterpret_cast<const f32x4*>(xt);
+    a.count = count, a.token_tiles = (count + 15) / 16;
+    a.params = params, a.q = q, a.kcache = kcache_layer, a.vcache = vcache_layer;
+    a.capacity = capacity;
+    return resident ? run_tile<K_F32, 3, EPI_QKV>(LH_QKV_ROWS, a, s)
+                    : run_tile<K_FP8, 3, EPI_QKV>(LH_QKV_ROWS, a, s);
+}
+
+extern "C" int lh_launch_gateup_tile(int resident, const void* Wgate, const void* Wup, float sg,
+    float su, const float* xt, uint32_t count, float* gated_xt, hipStream_t s)
+{
+    TileArgs a = {};
+    a.W = static_cast<const char*>(Wgate), a.W1 = static_cast<const char*>(Wup);
+    a.s0 = sg, a.s1 = su;
+    a.xt = reinterpret_cast<const f32x4*>(xt);
+    a.count = count, a.token_tiles = (count + 15) / 16;
+    a.gated = reinterpret_cast<f32x4*>(gated_xt);
+    return resident ? run_tile<K_F32, 3, EPI_GATEUP>(2 * LH_INNER, a, s)
+                    : run_tile<K_FP8, 3, EPI_GATEUP>(2 * LH_INNER, a, s);
+}
+
+extern "C" int lh_launch_residual_tile(int resident, const void* W, float scale, uint32_t cols,
+    const float* xt, uint32_t count, float* x, hipStream_t s)
+{
+    TileArgs a = {};
+    a.W = static_cast<const char*>(W);
+    a.s0 = scale;
+    a.xt = reinterpret_cast<const f32x4*>(xt);
+    a.count = count, a.token_tiles = (count + 15) / 16;
+    a.x = x;
+    if (cols == LH_QUERY) {
+        return resident ? run_tile<K_F32, 4, EPI_RESIDUAL>(LH_HIDDEN, a, s)
+                        : run_tile<K_FP8, 4, EPI_RESIDUAL>(LH_HIDDEN, a, s);
+    }
+    if (cols == LH_INNER) {
+        return resident ? run_tile<K_F32, 9, EPI_RESIDUAL>(LH_HIDDEN, a, s)
+                        : run_tile<K_FP8, 9, EPI_RESIDUAL>(LH_HIDDEN, a, s);
+    }
+    return -1;
+}
