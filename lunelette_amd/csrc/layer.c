@@ -328,10 +328,8 @@ static int layer_tiles(const lh_layer_weights *w, float *x, float *keys, float *
     if (launched(lh_launch_norm_tile(x, w->input_norm, ws->d_xn, n, s), "input norm") ||
         launched(lh_launch_qkv_tile(resident, wqkv, w->scale[0], w->scale[1], w->scale[2],
             ws->d_xn, ws->d_params, n, ws->d_q, keys, values, C, s), "qkv") ||
-        launched(lh_launch_attention(ws->d_q, keys, values, ws->d_params, (uint32_t)ws->length, n,
-            C, ws->d_PM, ws->d_PT, ws->d_PA, ws->d_arrive, ws->d_bflags, ++ws->epoch,
-            ws->handoff_fault, ws->d_attn, s), "attention") ||
-        launched(lh_launch_tile_rows(ws->d_attn, ws->d_up, n, s), "attention rows") ||
+        launched(lh_launch_attention_tiles(ws->d_q, keys, values, (uint32_t)ws->length, n, C,
+            ws->d_PM, ws->d_PT, ws->d_PA, ws->d_up, s), "attention") ||
         launched(lh_launch_residual_tile(resident, wo, w->scale[3], LH_QUERY, ws->d_up, n, x, s),
             "o") ||
         launched(lh_launch_norm_tile(x, w->post_norm, ws->d_xn, n, s), "post norm") ||

@@ -79,7 +79,9 @@ struct CombineShared {
 // group s of each 256-block round; every quarter recomputes M and the block
 // factors, so the four workgroups of a head are independent. Bitwise the
 // schedule above (the dims never mix; groups start at multiples of 8 from
-// block 0 and add left to right across rounds).
+// block 0 and add left to right across rounds). XT: out in the o projection's
+// activation tile order (lh_xt_word).
+template <bool XT = false>
 __device__ __forceinline__ void attn_combine(const float* __restrict__ PM,
     const float* __restrict__ PT, const float* __restrict__ PA, uint32_t n, uint32_t capacity,
     uint32_t h, uint32_t qd, uint32_t t, float* __restrict__ out, CombineShared& sh)
@@ -165,8 +167,9 @@ __device__ __forceinline__ void attn_combine(const float* __restrict__ PM,
         __syncthreads();
     }
     if (tid < 8) {
-        reinterpret_cast<float4*>(out + (size_t)t * LH_QUERY + h * LH_HEAD_DIM)[8 * qd + c] =
-            make_float4(A.x / T, A.y / T, A.z / T, A.w / T);
+        const uint32_t col = h * LH_HEAD_DIM + 32 * qd + 4 * c;
+        reinterpret_cast<float4*>(out)[XT ? lh_xt_word(t, col, LH_QUERY)
+            : ((size_t)t * LH_QUERY + col) / 4] = make_float4(A.x / T, A.y / T, A.z / T, A.w / T);
     }
 }
 

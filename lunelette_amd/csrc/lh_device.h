@@ -131,6 +131,27 @@ __device__ __forceinline__ float expf_cw(float x)
     return __builtin_ldexpf(p, (int)k);
 }
 
+// expf_cw without branches: the same bits, for callers whose lanes all need it.
+__device__ __forceinline__ float expf_flat(float x)
+{
+    const float c = fminf(fmaxf(x, -88.0f), 89.0f);   // NaN too; replaced below
+    const float k = __builtin_rintf(c * 1.44269502162933349609375f);
+    float r = __builtin_fmaf(k, -0.693145751953125f, c);
+    r = __builtin_fmaf(k, -1.428606765330187045037746429443359375e-06f, r);
+    float p = 1.98412698412698412698e-04f;
+    p = __builtin_fmaf(p, r, 1.38888888888888888889e-03f);
+    p = __builtin_fmaf(p, r, 8.33333333333333333333e-03f);
+    p = __builtin_fmaf(p, r, 4.16666666666666666667e-02f);
+    p = __builtin_fmaf(p, r, 1.66666666666666666667e-01f);
+    p = __builtin_fmaf(p, r, 0.5f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_ldexpf(p, (int)k);
+    p = x > 88.72283935546875f ? __builtin_inff() : p;
+    p = x < -87.33654022216796875f ? 0.0f : p;
+    return x != x ? x : p;
+}
+
 // SiLU v/(1+exp(-v)) (src/metal_kernels.metal:55-56) with the division
 // correctly rounded (hipcc's default fp32 division).
 __device__ __forceinline__ float silu(float v)
@@ -150,6 +171,16 @@ __device__ __forceinline__ size_t xs_at(uint32_t t, uint32_t c, uint32_t K)
 {
     return ((((size_t)(t >> 4) * (K >> 6) + (c >> 6)) * 2 + ((c >> 3) & 1)) << 9) +
         ((((c >> 4) & 3) * 16 + (t & 15)) << 3) + (c & 7);
+}
+
+// 16-byte word of (token t, columns col .. col + 3) in the activation tile
+// order of a K-column projection; col % 4 == 0. Tiles of 16 tokens; in a tile
+// [chunk][g][wave s][quad][block b][token % 16], col = 1024 chunk + 512 g +
+// 128 b + 16 s + 4 quad.
+__device__ __forceinline__ size_t lh_xt_word(uint32_t t, uint32_t col, uint32_t K)
+{
+    const uint32_t cg = col >> 9, b = (col >> 7) & 3, sq = (col >> 2) & 31;
+    return ((size_t)(t >> 4) * (K >> 9) + cg) * 2048 + sq * 64 + b * 16 + (t & 15);
 }
 
 // Token of workgroup w in a launch of one workgroup per token row (count

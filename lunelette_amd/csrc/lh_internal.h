@@ -26,7 +26,11 @@ int lh_launch_gateup_silu(int lookup, const uint8_t *Wgate, const uint8_t *Wup, 
  * never used). resident: FP32 weights, otherwise FP8 codes. */
 int lh_launch_norm_tile(const float *x, const float *gamma, float *xt, uint32_t count,
     hipStream_t s);
-int lh_launch_tile_rows(const float *x, float *xt, uint32_t count, hipStream_t s);
+/* Attention of several tokens (block partials and their combine), output in
+ * tile order. */
+int lh_launch_attention_tiles(const float *q, const float *kcache_layer,
+    const float *vcache_layer, uint32_t length, uint32_t count, uint32_t capacity, float *PM,
+    float *PT, float *PA, float *xt, hipStream_t s);
 int lh_launch_qkv_tile(int resident, const void *Wqkv, float sq, float sk, float sv,
     const float *xt, const lh_step_params *params, uint32_t count, float *q, float *kcache_layer,
     float *vcache_layer, uint32_t capacity, hipStream_t s);

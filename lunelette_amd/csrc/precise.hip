@@ -28,6 +28,7 @@
 // holds under this load). Measured there 0.61 ms (65 to 75% of that rate),
 // where the row dots it replaces, one token per workgroup, took 3.7 ms (each
 // token read and decoded every weight again: 16 TFLOP/s).
+#include "lh_attention_blocks.h"
 #include "lh_device.h"
 #include "lh_internal.h"
 
@@ -56,16 +57,6 @@ struct TileArgs {
     uint32_t capacity;
     f32x4* gated;          // EPI_GATEUP: lh_xt_word order, 9216 columns
 };
-
-// 16-byte word of (token t, columns col .. col + 3) in the activation tile
-// order of a K-column projection; col % 4 == 0. Tiles of 16 tokens; in a tile
-// [chunk][g][wave s][quad][block b][token % 16], col = 1024 chunk + 512 g +
-// 128 b + 16 s + 4 quad.
-__device__ __forceinline__ size_t lh_xt_word(uint32_t t, uint32_t col, uint32_t K)
-{
-    const uint32_t cg = col >> 9, b = (col >> 7) & 3, sq = (col >> 2) & 31;
-    return ((size_t)(t >> 4) * (K >> 9) + cg) * 2048 + sq * 64 + b * 16 + (t & 15);
-}
 
 // The weight rows of a workgroup's 16 RT tile rows n. EPI_RESIDUAL: consecutive
 // rows. EPI_QKV: the lower halves of 8 RT consecutive RoPE pairs of one head,
@@ -393,13 +384,308 @@ k_norm_tile(const float* __restrict__ x, const float* __restrict__ gamma, f32x4*
     xt[lh_xt_word(t, 4 * tid, LH_HIDDEN)] = y;
 }
 
-// Attention output rows of 4096 into the o projection's tile order. grid
-// (count), block 1024: thread i owns columns 4i .. 4i+3.
-__global__ void __launch_bounds__(1024)
-k_tile_rows(const f32x4* __restrict__ x, f32x4* __restrict__ xt)
+// The attention block partials of several tokens at once, bit for bit those of
+// attn_block (lh_attention_blocks.h). The 4 query heads of a kv head times 4
+// tokens are the 16 columns (query rows) of the products, one tile per wave.
+//   Scores, transposed: v_mfma_f32_16x16x1_4b with A = K (16 positions) and
+// B = Q; block c of the instruction is the chain c_c over dims 32c .. 32c + 31.
+// Lane l then holds, for query row l % 16, positions 16 pt + 4 (l / 16) + r.
+//   The maximum and the 64-position tree run over the lane's registers and
+// the four lane groups; a 4 x 4 transpose of registers and lane groups
+// (v_permlane32_swap, v_permlane16_swap) puts positions 4 st .. 4 st + 3 into
+// the lane groups of register st, in position order.
+//   P.V, transposed: v_mfma_f32_16x16x4_f32, whose four products add one after
+// the other, each rounded (k ascending), with A = V columns, B = P: the
+// canonical chain over the positions.
+// K and V come by direct loads to LDS, shared by the workgroup's four waves; the
+// next block's K is requested after the scores, its V after the chains.
+// Masked positions (past a token's own) carry e = 0: their products add +-0,
+// which can only turn a -0 sum into +0, and the combine's chain from +0 gives
+// the same bits for both. A nonfinite V among them would not be neutral: such
+// a block redoes its chains without them.
+// Bound: FP32 matrix instructions, 8192 cycles per wave and block: 256 tokens
+// after 4096 positions are 17.6 GFLOP, 0.13 ms at 2 GHz, and write 285 MB of
+// partials. Measured there 0.24 ms (0.76 ms with one token per workgroup,
+// k_attn_blocks) plus 0.06 ms for the combine, which reads the partials back
+// at 4.9 TB/s; 37 tokens after 777: 19 us plus 9 (30 and 5).
+//
+// grid 8 * query groups * ranges, block 256: id = (range * groups + group) * 8 +
+// kv head; a group is 16 tokens, a range `per` consecutive blocks.
+__global__ void __launch_bounds__(256, 2)
+k_attn_tiles(const float* __restrict__ q, const float* __restrict__ kcache,
+    const float* __restrict__ vcache, uint32_t length, uint32_t count, uint32_t capacity,
+    uint32_t groups, uint32_t per, float* __restrict__ PM, float* __restrict__ PT,
+    float* __restrict__ PA)
 {
-    const uint32_t t = blockIdx.x, tid = threadIdx.x;
-    xt[lh_xt_word(t, 4 * tid, LH_QUERY)] = x[(size_t)t * (LH_QUERY / 4) + tid];
+#ifdef __HIP_DEVICE_COMPILE__
+    constexpr uint32_t WORDS = LH_ATTN_BLOCK * LH_HEAD_DIM / 4;
+    __shared__ f32x4 ks[WORDS];
+    __shared__ f32x4 vs[WORDS];
+    const uint32_t kvh = blockIdx.x & 7, rest = blockIdx.x >> 3;
+    const uint32_t group = rest % groups, range = rest / groups;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t col = lane & 15, lg = lane >> 4;
+    // Blocks of this workgroup: up to its last token's position.
+    const uint32_t last = group * 16 + 15 < count ? group * 16 + 15 : count - 1;
+    const uint32_t need = (length + last) / LH_ATTN_BLOCK + 1;
+    const uint32_t b0 = range * per, b1 = b0 + per < need ? b0 + per : need;
+    if (b0 >= b1) {
+        return;
+    }
+    // Query row col: token t, head kvh * 4 + col % 4; rows past count repeat
+    // the last token, whose bits they store once more. A row also stores the
+    // partials of its group's blocks past its own last position, which no
+    // combine reads: every store is issued by every wave, so the waits below
+    // can count them.
+    const uint32_t tr = group * 16 + wave * 4 + (col >> 2), t = tr < count ? tr : count - 1;
+    const uint32_t n = length + t + 1;   // positions the row attends
+    const uint32_t nbc = capacity / LH_ATTN_BLOCK;
+    const size_t th = (size_t)t * LH_HEADS + kvh * 4 + (col & 3);
+    const float* const kh = kcache + lh_kv_index(capacity, 0, kvh, 0);
+    const float* const vh = vcache + lh_kv_index(capacity, 0, kvh, 0);
+    // K: LDS word (8 pt + i) * 64 + l holds dims 32 (l / 16) + 4i .. + 3 of position
+    // 16 pt + l % 16 (the tile's words in lane order). V: rows as they are.
+    auto load_k = [&](uint32_t b) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(kh + (size_t)b * 64 * LH_HEAD_DIM) +
+            wave * 512 + col * 4 + lg;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            __builtin_amdgcn_global_load_lds(p + i * 64, ks + (wave * 8 + i) * 64, 16, 0, 0);
+        }
+    };
+    auto load_v = [&](uint32_t b) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(vh + (size_t)b * 64 * LH_HEAD_DIM) +
+            wave * 512 + lane;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            __builtin_amdgcn_global_load_lds(p + i * 64, vs + (wave * 8 + i) * 64, 16, 0, 0);
+        }
+    };
+    f32x4 qr[8];
+    const f32x4* qp = reinterpret_cast<const f32x4*>(q + th * LH_HEAD_DIM) + lg * 8;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        qr[i] = qp[i];
+    }
+    load_k(b0);
+    load_v(b0);
+    __builtin_amdgcn_s_waitcnt(0);
+    // Barrier after this wave's LDS reads; direct loads stay in flight.
+    auto sync = [&]() {
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto swap32 = [](float& a, float& b) {   // a's lanes 32..63 <-> b's lanes 0..31
+        const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b),
+            false, false);
+        a = __uint_as_float(s[0]);
+        b = __uint_as_float(s[1]);
+    };
+    auto swap16 = [](float& a, float& b) {   // a's odd rows <-> b's even rows
+        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b),
+            false, false);
+        a = __uint_as_float(s[0]);
+        b = __uint_as_float(s[1]);
+    };
+    for (uint32_t b = b0; b < b1; b++) {
+        const uint32_t first = b * LH_ATTN_BLOCK;
+        const bool whole = first + LH_ATTN_BLOCK <= length + 1;   // for every token
+        const uint32_t valid = n > first ? (n - first < 64 ? n - first : 64) : 0;
+        // K has landed; V's eight loads and the ten stores of the block
+        // before, issued after it, may be in flight.
+        __builtin_amdgcn_s_waitcnt(0x4f72);
+        sync();
+        float e[4][4];
+#pragma unroll
+        for (int pt = 0; pt < 4; pt += 2) {
+            f32x16 c0 = {}, c1 = {};
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const f32x4 k0 = ks[(pt * 8 + i) * 64 + lane];
+                const f32x4 k1 = ks[(pt * 8 + 8 + i) * 64 + lane];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    c0 = __builtin_amdgcn_mfma_f32_16x16x1f32(k0[j], qr[i][j], c0, 0, 0, 0);
+                    c1 = __builtin_amdgcn_mfma_f32_16x16x1f32(k1[j], qr[i][j], c1, 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                e[pt][r] = ((c0[r] + c0[4 + r]) + (c0[8 + r] + c0[12 + r])) * LH_SCORE_SCALE;
+                e[pt + 1][r] = ((c1[r] + c1[4 + r]) + (c1[8 + r] + c1[12 + r])) * LH_SCORE_SCALE;
+            }
+        }
+        sync();   // every wave has read K
+        // (The last block requests itself again, unused.)
+        const uint32_t next = b + 1 < b1 ? b + 1 : b;
+        load_k(next);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!whole) {
+#pragma unroll
+            for (int pt = 0; pt < 4; pt++) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    if (16 * pt + 4 * lg + r >= valid) {
+                        e[pt][r] = -__builtin_inff();
+                    }
+                }
+            }
+        }
+        float m = e[0][0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) {
+            m = fmaxf(m, e[i >> 2][i & 3]);
+        }
+        float x = m, y = m;
+        swap32(x, y);
+        m = fmaxf(x, y);
+        x = m, y = m;
+        swap16(x, y);
+        m = fmaxf(x, y);
+#pragma unroll
+        for (int pt = 0; pt < 4; pt++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float v = expf_flat(e[pt][r] - m);
+                e[pt][r] = whole || 16 * pt + 4 * lg + r < valid ? v : 0.0f;
+            }
+        }
+        // T_b: the halving tree over positions (32, 16 by pt; 8, 4 by lane
+        // group; 2, 1 by register).
+        float u[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            u[r] = (e[0][r] + e[2][r]) + (e[1][r] + e[3][r]);
+            x = u[r], y = u[r];
+            swap32(x, y);
+            u[r] = x + y;
+            x = u[r], y = u[r];
+            swap16(x, y);
+            u[r] = x + y;
+        }
+        const float total = (u[0] + u[2]) + (u[1] + u[3]);
+        // Register e[pt][a] of lane group k: position 16 pt + 4a + k.
+#pragma unroll
+        for (int pt = 0; pt < 4; pt++) {
+            swap32(e[pt][0], e[pt][2]);
+            swap32(e[pt][1], e[pt][3]);
+            swap16(e[pt][0], e[pt][1]);
+            swap16(e[pt][2], e[pt][3]);
+        }
+        // V has landed; the ten stores and the next K may be in flight.
+        __builtin_amdgcn_s_waitcnt(0x4f72);
+        sync();
+        // A operand row i of tile (h, j): dim 64h + 4 ((i % 4) * 4 + i / 4) + j, so
+        // that a lane's results for fixed (h, r) are words 4r + lg: contiguous
+        // over the lane groups.
+        const uint32_t vw = (col & 3) * 4 + (col >> 2);
+        f32x4 o[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                o[h][j] = f32x4{};
+            }
+        }
+        bool redo = false;
+        if (whole) {
+#pragma unroll
+            for (int st = 0; st < 16; st++) {
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const f32x4 v = vs[(4 * st + lg) * 32 + 16 * h + vw];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        o[h][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], e[st >> 2][st & 3],
+                            o[h][j], 0, 0, 0);
+                    }
+                }
+            }
+        } else {
+            // Rows past the call's last token are stale: they enter as 0.
+            const uint32_t live = length + count - first;
+#pragma unroll
+            for (int st = 0; st < 16; st++) {
+                const uint32_t p = 4 * st + lg;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const f32x4 v = vs[p * 32 + 16 * h + vw];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float vj = p < live ? v[j] : 0.0f;
+                        redo = redo || (__float_as_uint(vj) & 0x7f800000u) == 0x7f800000u;
+                        o[h][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vj, e[st >> 2][st & 3],
+                            o[h][j], 0, 0, 0);
+                    }
+                }
+            }
+            if (__builtin_amdgcn_ballot_w64(redo)) {
+                // The chains over the row's own positions only.
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        o[h][j] = f32x4{};
+                    }
+                }
+#pragma unroll
+                for (int st = 0; st < 16; st++) {
+#pragma unroll 1
+                    for (uint32_t k = 0; k < 4; k++) {
+                        const uint32_t p = 4 * st + k;
+                        const float ep = __int_as_float(__builtin_amdgcn_ds_bpermute(
+                            4 * (16 * k + col), __float_as_int(e[st >> 2][st & 3])));
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+#pragma unroll
+                            for (int r = 0; r < 4; r++) {
+                                const f32x4 v = vs[p * 32 + 16 * h + 4 * r + lg];
+#pragma unroll
+                                for (int j = 0; j < 4; j++) {
+                                    o[h][j][r] = p < valid
+                                        ? __builtin_fmaf(ep, v[j], o[h][j][r]) : o[h][j][r];
+                                }
+                            }
+                        }
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        sync();   // every wave has read V
+        load_v(next);
+        __builtin_amdgcn_sched_barrier(0);
+        float* const pa = PA + (th * nbc + b) * LH_HEAD_DIM;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                reinterpret_cast<f32x4*>(pa)[16 * h + 4 * r + lg] =
+                    f32x4{o[h][0][r], o[h][1][r], o[h][2][r], o[h][3][r]};
+            }
+        }
+        PM[th * nbc + b] = m;
+        PT[th * nbc + b] = total;
+    }
+    // The unused direct loads land before the LDS is given back.
+    __builtin_amdgcn_s_waitcnt(0);
+#endif
+}
+
+// The combine of the block partials above (attn_combine), into the o
+// projection's tile order. grid (32 heads x 4 dimension quarters, count), block 256.
+__global__ void __launch_bounds__(256)
+k_combine_tiles(const float* __restrict__ PM, const float* __restrict__ PT,
+    const float* __restrict__ PA, uint32_t length, uint32_t capacity, float* __restrict__ out)
+{
+    __shared__ CombineShared sh;
+    const uint32_t t = blockIdx.y;
+    attn_combine<true>(PM, PT, PA, length + t + 1, capacity, blockIdx.x >> 2, blockIdx.x & 3, t,
+        out, sh);
 }
 
 }  // namespace lh
@@ -448,10 +734,24 @@ extern "C" int lh_launch_norm_tile(const float* x, const float* gamma, float* xt
     return launched();
 }
 
-extern "C" int lh_launch_tile_rows(const float* x, float* xt, uint32_t count, hipStream_t s)
+// Ranges: the query groups of the 8 kv heads times the ranges fill the 512
+// workgroups that two per CU (64 KB of LDS each) hold at once.
+extern "C" int lh_launch_attention_tiles(const float* q, const float* kcache_layer,
+    const float* vcache_layer, uint32_t length, uint32_t count, uint32_t capacity, float* PM,
+    float* PT, float* PA, float* xt, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_tile_rows, dim3(count), dim3(1024), 0, s,
-        reinterpret_cast<const f32x4*>(x), reinterpret_cast<f32x4*>(xt));
+    if (!count || capacity % LH_ATTN_BLOCK || length + count > capacity) {
+        return -1;
+    }
+    const uint32_t groups = (count + 15) / 16, nblk = lh_attention_blocks(length, count);
+    const uint32_t ranges = groups < 64 ? 64 / groups : 1, per = (nblk + ranges - 1) / ranges;
+    hipLaunchKernelGGL(k_attn_tiles, dim3(8 * groups * ((nblk + per - 1) / per)), dim3(256), 0, s,
+        q, kcache_layer, vcache_layer, length, count, capacity, groups, per, PM, PT, PA);
+    if (launched()) {
+        return -1;
+    }
+    hipLaunchKernelGGL(k_combine_tiles, dim3(LH_HEADS * 4, count), dim3(256), 0, s, PM, PT, PA,
+        length, capacity, xt);
     return launched();
 }
 

@@ -124,6 +124,24 @@ def test_multi_token_layer_tiles(gpu, layer_host, length, count):
                 paths + [lh.PATH_LOOKUP] if count < 20 else paths)
 
 
+@pytest.mark.parametrize("length,count", [(0, 5), (70, 20), (120, 41)])
+def test_multi_token_layer_nonfinite_token(gpu, layer_host, length, count):
+    """A token whose input is infinite leaves NaN values in the cache; the
+    tokens before it, in the same attention block, must not see them, as in the
+    token-by-token path."""
+    x = syn.normal_f32(SEED, 9011, count * 3072).reshape(count, 3072)
+    x[count // 2, 7] = np.inf
+    kpm = syn.normal_f32(SEED, 9012, length * 1024).reshape(length, 1024)
+    vpm = syn.normal_f32(SEED, 9013, length * 1024).reshape(length, 1024)
+    got, want = (run_layer(gpu, layer_host, x.reshape(-1), kpm, vpm, length, count, 4352, path,
+                           False) for path in (lh.PATH_FUSED, lh.PATH_UNFUSED))
+    rows = np.isfinite(want[0].reshape(count, 3072)).all(axis=1)
+    assert rows[:count // 2].all() and not rows[count // 2:].any()
+    for g, w, name in zip(got, want, ("x", "k", "v")):
+        assert np.array_equal(np.isnan(g), np.isnan(w)), name
+        assert np.array_equal(bits(g)[~np.isnan(w)], bits(w)[~np.isnan(w)]), name
+
+
 def attention_on_device(gpu, q, kpm, vpm, length, count, capacity):
     ws = gpu.lh_workspace_create(capacity, count)
     assert ws, lh.last_error()
