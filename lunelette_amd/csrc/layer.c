@@ -237,59 +237,60 @@ static int launched(int status, const char *what)
     return 0;
 }
 
-/* Separate-operator path (also the resident FP32 strategy): every operator is
- * its own kernel, every row dot follows the same canonical schedule as the
- * fused kernels, so results are bitwise identical. */
+/* Separate-operator path: every operator is its own kernel, every row dot
+ * follows the same canonical schedule as the fused kernels, so results are
+ * bitwise identical. */
 static int layer_unfused(const lh_layer_weights *w, float *x, float *keys, float *values,
-    lh_workspace *ws, int resident, hipStream_t s)
+    lh_workspace *ws, hipStream_t s)
 {
     const uint32_t n = (uint32_t)ws->count, C = (uint32_t)ws->capacity;
-    const int kind = resident ? 2 : 0;
-    const void *wq = resident ? (const void *)w->f32_qkv : (const void *)w->qkv;
-    const size_t esize = resident ? 4 : 1;
-    const char *base = (const char *)wq;
-    const void *wk = base + (size_t)LH_QUERY * LH_HIDDEN * esize;
-    const void *wv = base + (size_t)(LH_QUERY + LH_KV) * LH_HIDDEN * esize;
-    const void *wo = resident ? (const void *)w->f32_o : (const void *)w->o;
-    const void *wg = resident ? (const void *)w->f32_gate : (const void *)w->gate;
-    const void *wu = resident ? (const void *)w->f32_up : (const void *)w->up;
-    const void *wd = resident ? (const void *)w->f32_down : (const void *)w->down;
+    const uint8_t *wk = w->qkv + (size_t)LH_QUERY * LH_HIDDEN;
+    const uint8_t *wv = w->qkv + (size_t)(LH_QUERY + LH_KV) * LH_HIDDEN;
     const lh_step_params *params = ws->d_params;
     if (launched(lh_launch_rmsnorm(w->input_norm, x, ws->d_xn, LH_HIDDEN, n, s), "input norm") ||
-        launched(lh_launch_matvec(kind, 0, wq, w->scale[0], ws->d_xn, ws->d_qraw, NULL,
+        launched(lh_launch_matvec(0, 0, w->qkv, w->scale[0], ws->d_xn, ws->d_qraw, NULL,
             LH_QUERY, LH_HIDDEN, n, s), "q") ||
-        launched(lh_launch_matvec(kind, 0, wk, w->scale[1], ws->d_xn, ws->d_kraw, NULL,
+        launched(lh_launch_matvec(0, 0, wk, w->scale[1], ws->d_xn, ws->d_kraw, NULL,
             LH_KV, LH_HIDDEN, n, s), "k") ||
-        launched(lh_launch_matvec(kind, 0, wv, w->scale[2], ws->d_xn, ws->d_vraw, NULL,
+        launched(lh_launch_matvec(0, 0, wv, w->scale[2], ws->d_xn, ws->d_vraw, NULL,
             LH_KV, LH_HIDDEN, n, s), "v") ||
         launched(lh_launch_rope_append(ws->d_qraw, ws->d_kraw, ws->d_vraw, params, n, ws->d_q,
             keys, values, C, s), "rope/append") ||
         launched(lh_launch_attention(ws->d_q, keys, values, ws->d_params, (uint32_t)ws->length, n,
             C, ws->d_PM, ws->d_PT, ws->d_PA, ws->d_arrive, ws->d_bflags, ++ws->epoch,
             ws->handoff_fault, ws->d_attn, s), "attention") ||
-        launched(lh_launch_matvec(kind, 0, wo, w->scale[3], ws->d_attn, x, x, LH_HIDDEN,
+        launched(lh_launch_matvec(0, 0, w->o, w->scale[3], ws->d_attn, x, x, LH_HIDDEN,
             LH_QUERY, n, s), "o") ||
         launched(lh_launch_rmsnorm(w->post_norm, x, ws->d_xn, LH_HIDDEN, n, s), "post norm") ||
-        launched(lh_launch_matvec(kind, 0, wg, w->scale[4], ws->d_xn, ws->d_gated, NULL,
+        launched(lh_launch_matvec(0, 0, w->gate, w->scale[4], ws->d_xn, ws->d_gated, NULL,
             LH_INNER, LH_HIDDEN, n, s), "gate") ||
-        launched(lh_launch_matvec(kind, 0, wu, w->scale[5], ws->d_xn, ws->d_up, NULL,
+        launched(lh_launch_matvec(0, 0, w->up, w->scale[5], ws->d_xn, ws->d_up, NULL,
             LH_INNER, LH_HIDDEN, n, s), "up") ||
         launched(lh_launch_silu_mul(ws->d_gated, ws->d_up, ws->d_gated, (size_t)n * LH_INNER, s),
             "silu") ||
-        launched(lh_launch_matvec(kind, 0, wd, w->scale[6], ws->d_gated, x, x, LH_HIDDEN,
+        launched(lh_launch_matvec(0, 0, w->down, w->scale[6], ws->d_gated, x, x, LH_HIDDEN,
             LH_INNER, n, s), "down")) {
         return -1;
     }
     return 0;
 }
 
+/* strategy: LH_ROWS_*, which weights and how they are decoded. */
 static int layer_fused(const lh_layer_weights *w, float *x, float *keys, float *values,
-    lh_workspace *ws, int lookup, hipStream_t s)
+    lh_workspace *ws, int strategy, hipStream_t s)
 {
     const uint32_t n = (uint32_t)ws->count, C = (uint32_t)ws->capacity;
     const lh_step_params *params = ws->d_params;
-    /* One decode token: q|k|v and the attention blocks share a launch. */
-    const int chained = n == 1 && lh_attention_chained((uint32_t)ws->length);
+    const int resident = strategy == LH_ROWS_F32, lookup = strategy == LH_ROWS_FP8_LOOKUP;
+    const int kind = resident ? 2 : 0;
+    const void *wqkv = resident ? (const void *)w->f32_qkv : (const void *)w->qkv;
+    const void *wo = resident ? (const void *)w->f32_o : (const void *)w->o;
+    const void *wg = resident ? (const void *)w->f32_gate : (const void *)w->gate;
+    const void *wu = resident ? (const void *)w->f32_up : (const void *)w->up;
+    const void *wd = resident ? (const void *)w->f32_down : (const void *)w->down;
+    /* One decode token on FP8 weights: q|k|v and the attention blocks share a
+     * launch. */
+    const int chained = n == 1 && !resident && lh_attention_chained((uint32_t)ws->length);
     if ((chained ?
             launched(lh_launch_qkv_attention(lookup, w->qkv, w->scale[0], w->scale[1],
                 w->scale[2], w->input_norm, x, params, (uint32_t)ws->length, ws->d_q, keys,
@@ -297,16 +298,16 @@ static int layer_fused(const lh_layer_weights *w, float *x, float *keys, float *
                 ws->d_arrive + FLAGS_WORD(ws->block), ws->d_bflags, ++ws->epoch,
                 ws->handoff_fault, ws->d_attn, s),
                 "qkv/attention") :
-            launched(lh_launch_qkv_rope(lookup, w->qkv, w->scale[0], w->scale[1], w->scale[2],
+            launched(lh_launch_qkv_rope(strategy, wqkv, w->scale[0], w->scale[1], w->scale[2],
                 w->input_norm, x, params, n, ws->d_q, keys, values, C, s), "qkv") ||
             launched(lh_launch_attention(ws->d_q, keys, values, ws->d_params,
                 (uint32_t)ws->length, n, C, ws->d_PM, ws->d_PT, ws->d_PA, ws->d_arrive,
                 ws->d_bflags, ++ws->epoch, ws->handoff_fault, ws->d_attn, s), "attention")) ||
-        launched(lh_launch_matvec(0, lookup, w->o, w->scale[3], ws->d_attn, x, x, LH_HIDDEN,
+        launched(lh_launch_matvec(kind, lookup, wo, w->scale[3], ws->d_attn, x, x, LH_HIDDEN,
             LH_QUERY, n, s), "o") ||
-        launched(lh_launch_gateup_silu(lookup, w->gate, w->up, w->scale[4], w->scale[5],
+        launched(lh_launch_gateup_silu(strategy, wg, wu, w->scale[4], w->scale[5],
             w->post_norm, x, n, ws->d_gated, s), "gate/up") ||
-        launched(lh_launch_matvec(0, lookup, w->down, w->scale[6], ws->d_gated, x, x, LH_HIDDEN,
+        launched(lh_launch_matvec(kind, lookup, wd, w->scale[6], ws->d_gated, x, x, LH_HIDDEN,
             LH_INNER, n, s), "down")) {
         return -1;
     }
@@ -392,19 +393,20 @@ int lh_layer_forward(const lh_layer_weights *w, float *d_x, float *d_keys, float
     const int tiles = ws->count >= (path == LH_PATH_RESIDENT ? TILES_MIN_RESIDENT : TILES_MIN);
     switch (path) {
     case LH_PATH_FUSED:
-        return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 0, s) : layer_fused(w, d_x, d_keys, d_values, ws, 0, s);
+        return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 0, s)
+                     : layer_fused(w, d_x, d_keys, d_values, ws, LH_ROWS_FP8, s);
     case LH_PATH_LOOKUP:
-        return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 0, s) :
-            layer_fused(w, d_x, d_keys, d_values, ws, 1, s);
+        return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 0, s)
+                     : layer_fused(w, d_x, d_keys, d_values, ws, LH_ROWS_FP8_LOOKUP, s);
     case LH_PATH_UNFUSED:
-        return layer_unfused(w, d_x, d_keys, d_values, ws, 0, s);
+        return layer_unfused(w, d_x, d_keys, d_values, ws, s);
     case LH_PATH_RESIDENT:
         if (!w->f32_qkv || !w->f32_o || !w->f32_gate || !w->f32_up || !w->f32_down) {
             lh_set_error("layer_forward: resident path needs FP32 weights");
             return -1;
         }
-        return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 1, s) :
-            layer_unfused(w, d_x, d_keys, d_values, ws, 1, s);
+        return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 1, s)
+                     : layer_fused(w, d_x, d_keys, d_values, ws, LH_ROWS_F32, s);
     case LH_PATH_MFMA:
         return lh_layer_forward_mfma(w, d_x, d_keys, d_values, ws, 0, NULL, s);
     default:

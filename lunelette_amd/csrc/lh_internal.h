@@ -16,11 +16,13 @@ extern "C" {
 /* kind: 0 FP8 codes (scaled), 1 BF16, 2 FP32. residual may be NULL. */
 int lh_launch_matvec(int kind, int lookup, const void *W, float scale, const float *x, float *y,
     const float *residual, uint32_t rows, uint32_t cols, uint32_t tokens, hipStream_t s);
-int lh_launch_qkv_rope(int lookup, const uint8_t *Wqkv, float sq, float sk, float sv,
+/* Weight rows of the fused decode kernels. */
+enum { LH_ROWS_FP8 = 0, LH_ROWS_FP8_LOOKUP = 1, LH_ROWS_F32 = 2 };
+int lh_launch_qkv_rope(int strategy, const void *Wqkv, float sq, float sk, float sv,
     const float *gamma, const float *x, const lh_step_params *params, uint32_t count,
     float *q, float *kcache_layer, float *vcache_layer, uint32_t capacity, hipStream_t s);
-int lh_launch_gateup_silu(int lookup, const uint8_t *Wgate, const uint8_t *Wup, float sg,
-    float su, const float *gamma, const float *x, uint32_t count, float *gated, hipStream_t s);
+int lh_launch_gateup_silu(int strategy, const void *Wgate, const void *Wup, float sg, float su,
+    const float *gamma, const float *x, uint32_t count, float *gated, hipStream_t s);
 /* Multi-token projections on the FP32 matrix instructions (precise.hip); xt:
  * activations in tile order, whole 16-token tiles (rows past count are read,
  * never used). resident: FP32 weights, otherwise FP8 codes. */

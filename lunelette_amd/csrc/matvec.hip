@@ -6,6 +6,14 @@
 // across all its chunks, and the 64 lane sums reduce by one fixed tree. The
 // per-tensor scale multiplies the row total once.
 //
+// FP32 rows (the resident strategy) would put 64 bytes between a load's lanes
+// and fetch every line four times over (3.3 TB/s of rows); their loads are
+// contiguous instead, 16 bytes per lane, and the accumulators of a chain visit
+// the four lanes that hold its columns (dot_f32): 64 instead of 16 fused
+// multiply-adds per lane and chunk, a fifth of what the memory rate leaves room
+// for. Bound: HBM; gate/up (226 MB) 68 -> 35 us (6.4 TB/s), down (113 MB) 32
+// -> 19 us, the whole layer after 1023 positions 204 -> 87 us.
+//
 // One wave owns whole rows. The workgroup stages the input row once in LDS;
 // where a norm precedes the projection (q|k|v, gate/up, head) the workgroup
 // applies the canonical RMSNorm there before any dot. The q|k|v and gate/up
@@ -37,6 +45,24 @@ __device__ __forceinline__ void load_w(WVec<KIND>& w, const void* base, size_t r
 #pragma unroll
     for (int i = 0; i < (int)(sizeof(WVec<KIND>) / 16); i++) {
         w.v[i] = __builtin_nontemporal_load(p + i);
+    }
+}
+
+// One chunk of a row of K columns into w: the lane's own 16 columns, or (FP32)
+// the chunk's 16-byte words 64 i + lane.
+template <int KIND>
+__device__ __forceinline__ void load_chunk(WVec<KIND>& w, const void* base, size_t row, uint32_t K,
+    int c, int lane)
+{
+    if constexpr (KIND == K_F32) {
+        const u32x4* p = reinterpret_cast<const u32x4*>(
+            static_cast<const float*>(base) + row * K + c * LH_CHUNK) + lane;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            w.v[i] = __builtin_nontemporal_load(p + 64 * i);
+        }
+    } else {
+        load_w<KIND>(w, base, row, K, c * LH_CHUNK + lane * LH_LANE_COLS);
     }
 }
 
@@ -152,13 +178,14 @@ __device__ __forceinline__ void stage_load(const float* row, float4 (&xv)[NCH])
     }
 }
 
-template <int NCH>
+// LINEAR (FP32 weight rows): word w of the row at xl[w].
+template <int NCH, bool LINEAR = false>
 __device__ __forceinline__ void stage_commit(const float4 (&xv)[NCH], float4* xl)
 {
     const uint32_t tid = threadIdx.x;
 #pragma unroll
     for (int i = 0; i < NCH; i++) {
-        xl[staged_word(i, tid)] = xv[i];
+        xl[LINEAR ? tid + 256 * i : staged_word(i, tid)] = xv[i];
     }
     __syncthreads();
 }
@@ -168,8 +195,9 @@ __device__ __forceinline__ void stage_commit(const float4 (&xv)[NCH], float4* xl
 // columns 2h, 2h+1, half h&1 of 16-byte word h/2), so every thread count that
 // divides 1536 needs no guards. norm_commit stores the units in the LDS layout
 // above; wave 0 forms the canonical r from LDS; every thread then writes
-// gamma * (x * r) over its own units. Three barriers; the last one publishes the
-// normalized row (and anything else the workgroup stored before it).
+// gamma * (x * r) over its own units (LINEAR: unit h at 8-byte word h). Three
+// barriers; the last one publishes the normalized row (and anything else the
+// workgroup stored before it).
 template <int T>
 __device__ __forceinline__ void norm_load(const float* row, const float* gamma,
     float2 (&xv)[1536 / T], float2 (&gv)[1536 / T])
@@ -189,7 +217,7 @@ __device__ __forceinline__ float2* staged_unit(float4* xl, uint32_t h)
     return reinterpret_cast<float2*>(xl + staged_word(w >> 8, w & 255)) + (h & 1);
 }
 
-template <int T>
+template <int T, bool LINEAR = false>
 __device__ __forceinline__ void norm_commit(const float2 (&xv)[1536 / T],
     const float2 (&gv)[1536 / T], float4* xl, float* r_s)
 {
@@ -218,7 +246,9 @@ __device__ __forceinline__ void norm_commit(const float2 (&xv)[1536 / T],
     const float r = *r_s;
 #pragma unroll
     for (int u = 0; u < 1536 / T; u++) {
-        *staged_unit(xl, tid + T * u) = make_float2(gv[u].x * (xv[u].x * r), gv[u].y * (xv[u].y * r));
+        float2* const unit = LINEAR ? reinterpret_cast<float2*>(xl) + tid + T * u
+                                    : staged_unit(xl, tid + T * u);
+        *unit = make_float2(gv[u].x * (xv[u].x * r), gv[u].y * (xv[u].y * r));
     }
     __syncthreads();
 }
@@ -236,8 +266,66 @@ __device__ __forceinline__ void issue_rows(const void* W, const uint32_t (&rows)
     for (int r = 0; r < R; r++) {
 #pragma unroll
         for (int c = 0; c < NCH; c++) {
-            load_w<KIND>(wv[r][c], W, rows[r], K, c * LH_CHUNK + lane * LH_LANE_COLS);
+            load_chunk<KIND>(wv[r][c], W, rows[r], K, c, lane);
         }
+    }
+}
+
+// R canonical dots of FP32 rows loaded as load_chunk does, x staged linearly.
+// Word 64 i + l holds columns 4 (l % 4) .. + 3 of chain 16 i + l / 4, so a
+// chain's accumulator starts in lane l % 4 = 0 of its quad, runs four columns
+// there and moves to the next lane (a quad rotation), four times per chunk;
+// the other three accumulators of a quad are never used. The tree's distances
+// 32 and 16 then lie between the registers i, 8 .. 1 between lanes 32, 16, 8
+// and 4 apart.
+template <int NCH, int R>
+__device__ __forceinline__ void dot_f32(const WVec<K_F32> (&wv)[R][NCH], const float4* xl,
+    float (&out)[R])
+{
+    const uint32_t lane = threadIdx.x & 63;
+    float acc[R][4];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            acc[r][i] = 0.0f;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NCH; c++) {
+        float4 x[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            x[i] = xl[c * 256 + i * 64 + lane];
+        }
+#pragma unroll
+        for (int step = 0; step < 4; step++) {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const u32x4 w = wv[r][c].v[i];
+                    float a = acc[r][i];
+                    a = __builtin_fmaf(__uint_as_float(w.x), x[i].x, a);
+                    a = __builtin_fmaf(__uint_as_float(w.y), x[i].y, a);
+                    a = __builtin_fmaf(__uint_as_float(w.z), x[i].z, a);
+                    a = __builtin_fmaf(__uint_as_float(w.w), x[i].w, a);
+                    acc[r][i] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0x93,
+                        0xf, 0xf, false));   // quad_perm [3,0,1,2]
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        float v = (acc[r][0] + acc[r][2]) + (acc[r][1] + acc[r][3]);
+        const uint32_t u = __float_as_uint(v);
+        v = v + __uint_as_float(__builtin_amdgcn_permlane32_swap(u, u, false, false)[1]);
+        const uint32_t w = __float_as_uint(v);
+        v = v + __uint_as_float(__builtin_amdgcn_permlane16_swap(w, w, false, false)[1]);
+        v = v + dpp_row_shl(v, 8);
+        v = v + dpp_row_shl(v, 4);
+        out[r] = v;
     }
 }
 
@@ -249,6 +337,10 @@ template <int KIND, bool LUT, int NCH, int R>
 __device__ __forceinline__ void dot_rows(const WVec<KIND> (&wv)[R][NCH], const float4* xl,
     const float* lut, float (&out)[R])
 {
+    if constexpr (KIND == K_F32) {
+        dot_f32<NCH, R>(wv, xl, out);
+        return;
+    }
     const uint32_t lane = threadIdx.x & 63;
     float acc[R];
 #pragma unroll
@@ -297,7 +389,7 @@ struct RowStream {
         const int lane = threadIdx.x & 63;
 #pragma unroll
         for (int c = 0; c < NCH; c++) {
-            load_w<KIND>(wv[slot][c], W, row, NCH * LH_CHUNK, c * LH_CHUNK + lane * LH_LANE_COLS);
+            load_chunk<KIND>(wv[slot][c], W, row, NCH * LH_CHUNK, c, lane);
         }
     }
 
@@ -352,11 +444,11 @@ k_rows(const void* __restrict__ W, float scale, const float* __restrict__ x, flo
     for (int r = 0; r < R; r++) {
         rr[r] = row0 + r;
     }
-    // FP8 rows stream with one row of loads in flight ahead of the row being
-    // dotted (RowStream); with all R rows requested at once the model's o
-    // and down projections ran 6% and 8% slower. Other kinds keep every row
-    // in flight.
-    constexpr bool STREAM = KIND == K_FP8 && R > 1;
+    // FP8 and FP32 rows stream with one row of loads in flight ahead of the row
+    // being dotted (RowStream); with all R rows requested at once the model's
+    // FP8 o and down projections ran 6% and 8% slower. BF16 rows are all in
+    // flight.
+    constexpr bool STREAM = KIND != K_BF16 && R > 1;
     RowStream<KIND, NCH, R, 1> stream;
     WVec<KIND> wv[STREAM ? 1 : R][NCH];
     if constexpr (STREAM) {
@@ -364,7 +456,7 @@ k_rows(const void* __restrict__ W, float scale, const float* __restrict__ x, flo
     } else {
         issue_rows<KIND, NCH, R>(W, rr, wv);
     }
-    stage_commit<NCH>(xv, xin_s);
+    stage_commit<NCH, KIND == K_F32>(xv, xin_s);
     // The epilogue's residual values are requested now, after the row is
     // staged, so they return behind the weights instead of costing a memory
     // round trip after the dots. Written as assembly because the compiler
@@ -482,8 +574,8 @@ __device__ __forceinline__ uint32_t qkv_pair(uint32_t g, uint32_t kvh, uint32_t 
         : li < 320 ? (32 + kvh) * 64 + (li - 256) : (40 + kvh) * 64 + (li - 320);
 }
 
-template <bool LUT, bool BYKV>
-__device__ __forceinline__ void qkv_rope_body(const uint8_t* __restrict__ Wqkv, float3 scales,
+template <int KIND, bool LUT, bool BYKV>
+__device__ __forceinline__ void qkv_rope_body(const void* __restrict__ Wqkv, float3 scales,
     const float* __restrict__ gamma, const float* __restrict__ xin,
     const lh_step_params* __restrict__ params, float* __restrict__ qout,
     float* __restrict__ kcache, float* __restrict__ vcache, uint32_t capacity, uint32_t g,
@@ -506,11 +598,11 @@ __device__ __forceinline__ void qkv_rope_body(const uint8_t* __restrict__ Wqkv, 
         const uint32_t pair = qkv_pair<BYKV>(g, kvh, k0 + j);
         rr[j] = (pair >> 6) * 128 + (pair & 63) + (upper ? 64 : 0);
     }
-    WVec<K_FP8> wv[3][3];
-    issue_rows<K_FP8, 3, 3>(Wqkv, rr, wv);
-    norm_commit<T>(xv, gv, sh.xin, &sh.r);
+    WVec<KIND> wv[3][3];
+    issue_rows<KIND, 3, 3>(Wqkv, rr, wv);
+    norm_commit<T, KIND == K_F32>(xv, gv, sh.xin, &sh.r);
     float dots[3];
-    dot_rows<K_FP8, LUT, 3, 3>(wv, sh.xin, sh.lut, dots);
+    dot_rows<KIND, LUT, 3, 3>(wv, sh.xin, sh.lut, dots);
     if (lane == 0) {
 #pragma unroll
         for (int j = 0; j < 3; j++) {
@@ -549,16 +641,16 @@ __device__ __forceinline__ void qkv_rope_body(const uint8_t* __restrict__ Wqkv, 
 }
 
 // grid (512, count), block 256: workgroup x owns pairs 6x .. 6x+5.
-template <bool LUT>
+template <int KIND, bool LUT>
 __global__ void __launch_bounds__(256)
-k_qkv_rope(const uint8_t* __restrict__ Wqkv, float3 scales, const float* __restrict__ gamma,
+k_qkv_rope(const void* __restrict__ Wqkv, float3 scales, const float* __restrict__ gamma,
     const float* __restrict__ xin, const lh_step_params* __restrict__ params,
     float* __restrict__ qout, float* __restrict__ kcache, float* __restrict__ vcache,
     uint32_t capacity)
 {
     __shared__ QkvShared<LUT> sh;
-    qkv_rope_body<LUT, false>(Wqkv, scales, gamma, xin, params, qout, kcache, vcache, capacity,
-        blockIdx.x, 0, blockIdx.y, sh);
+    qkv_rope_body<KIND, LUT, false>(Wqkv, scales, gamma, xin, params, qout, kcache, vcache,
+        capacity, blockIdx.x, 0, blockIdx.y, sh);
 }
 
 // One decode token's q|k|v projection and attention blocks in one launch
@@ -605,7 +697,7 @@ k_qkv_attn(const uint8_t* __restrict__ Wqkv, float3 scales, const float* __restr
         return;
     }
     if (blockIdx.x < 8 * QKV_PRODUCERS) {
-        qkv_rope_body<LUT, true>(Wqkv, scales, gamma, xin, params, qout, kcache, vcache,
+        qkv_rope_body<K_FP8, LUT, true>(Wqkv, scales, gamma, xin, params, qout, kcache, vcache,
             capacity, blockIdx.x >> 3, kvh, 0, sh.qkv);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the rows are in L2
         __syncthreads();
@@ -627,11 +719,10 @@ k_qkv_attn(const uint8_t* __restrict__ Wqkv, float3 scales, const float* __restr
 // flight. The scaled dots meet in LDS, where threads 0..35 form
 // SiLU(gate)*up. grid (9216/36, count), block 512.
 constexpr int GATEUP_ROWS = 9;  // rows per wave
-constexpr int GATEUP_DEPTH = 3; // rows of loads in flight per wave
 
-template <bool LUT>
+template <int KIND, bool LUT>
 __global__ void __launch_bounds__(512)
-k_gateup_silu(const uint8_t* __restrict__ Wgate, const uint8_t* __restrict__ Wup, float2 scales,
+k_gateup_silu(const void* __restrict__ Wgate, const void* __restrict__ Wup, float2 scales,
     const float* __restrict__ gamma, const float* __restrict__ xin, float* __restrict__ gated)
 {
     constexpr int T = 512;
@@ -648,7 +739,7 @@ k_gateup_silu(const uint8_t* __restrict__ Wgate, const uint8_t* __restrict__ Wup
     const uint32_t t = blockIdx.y;
     const bool up = wave >= 4;
     const uint32_t k0 = GATEUP_ROWS * (wave & 3);
-    const uint8_t* W = up ? Wup : Wgate;
+    const void* W = up ? Wup : Wgate;
     uint32_t rr[GATEUP_ROWS];
 #pragma unroll
     for (int r = 0; r < GATEUP_ROWS; r++) {
@@ -656,9 +747,10 @@ k_gateup_silu(const uint8_t* __restrict__ Wgate, const uint8_t* __restrict__ Wup
     }
     float2 xv[1536 / T], gv[1536 / T];
     norm_load<T>(xin + (size_t)t * LH_HIDDEN, gamma, xv, gv);
-    RowStream<K_FP8, 3, GATEUP_ROWS, GATEUP_DEPTH> stream;
+    // Rows of loads in flight per wave: 9 KB of FP8, 24 KB of FP32.
+    RowStream<KIND, 3, GATEUP_ROWS, KIND == K_F32 ? 2 : 3> stream;
     stream.start(W, rr);
-    norm_commit<T>(xv, gv, xin_s, &r_s);
+    norm_commit<T, KIND == K_F32>(xv, gv, xin_s, &r_s);
     float dots[GATEUP_ROWS];
     stream.template run<LUT>(W, rr, xin_s, lut_s, dots);
     if (lane == 0) {
@@ -755,23 +847,23 @@ static int launch_rows(const void* W, float scale, const float* x, float* y, con
 }
 
 
-// Model shapes (3072, 4096 or 9216 columns) use the unrolled kernel. FP8 and
-// BF16 weights take three rows per wave where the row count allows it (the
-// model's 3072-row o and down projections then give each SIMD of the 256 CUs
-// the same work); resident FP32 rows take fewer to fit the register file.
+// Model shapes (3072, 4096 or 9216 columns) use the unrolled kernel, three
+// rows per wave where the row count allows it (the model's 3072-row o and
+// down projections then give each SIMD of the 256 CUs the same work); FP32
+// rows of 9216 columns take one, all of whose loads fit the register file.
 // Returns 1 when the shape is not a model shape.
 template <int KIND, bool LUT>
 static int launch_model_rows(const void* W, float scale, const float* x, float* y,
     const float* residual, uint32_t rows, uint32_t cols, uint32_t tokens, hipStream_t s)
 {
-    if constexpr (KIND != K_F32) {
-        if (rows % 12 == 0) {
-            if (cols == 3072) {
-                return launch_rows<KIND, LUT, 3, 3>(W, scale, x, y, residual, rows, tokens, s);
-            }
-            if (cols == 4096) {
-                return launch_rows<KIND, LUT, 4, 3>(W, scale, x, y, residual, rows, tokens, s);
-            }
+    if (rows % 12 == 0) {
+        if (cols == 3072) {
+            return launch_rows<KIND, LUT, 3, 3>(W, scale, x, y, residual, rows, tokens, s);
+        }
+        if (cols == 4096) {
+            return launch_rows<KIND, LUT, 4, 3>(W, scale, x, y, residual, rows, tokens, s);
+        }
+        if constexpr (KIND != K_F32) {
             if (cols == 9216) {
                 return launch_rows<KIND, LUT, 9, 3>(W, scale, x, y, residual, rows, tokens, s);
             }
@@ -836,19 +928,22 @@ extern "C" int lh_launch_matvec(int kind, int lookup, const void* W, float scale
     return -1;
 }
 
-extern "C" int lh_launch_qkv_rope(int lookup, const uint8_t* Wqkv, float sq, float sk, float sv,
+extern "C" int lh_launch_qkv_rope(int strategy, const void* Wqkv, float sq, float sk, float sv,
     const float* gamma, const float* x, const lh_step_params* params, uint32_t count,
     float* q, float* kcache_layer, float* vcache_layer, uint32_t capacity, hipStream_t s)
 {
     dim3 grid(48 * 64 / 6, count);
     float3 scales = make_float3(sq, sk, sv);
-    if (lookup) {
-        hipLaunchKernelGGL(k_qkv_rope<true>, grid, dim3(256), 0, s, Wqkv, scales, gamma, x, params,
-            q, kcache_layer, vcache_layer, capacity);
+#define LH_QKV(K, L) hipLaunchKernelGGL((k_qkv_rope<K, L>), grid, dim3(256), 0, s, Wqkv, scales, \
+        gamma, x, params, q, kcache_layer, vcache_layer, capacity)
+    if (strategy == LH_ROWS_F32) {
+        LH_QKV(K_F32, false);
+    } else if (strategy == LH_ROWS_FP8_LOOKUP) {
+        LH_QKV(K_FP8, true);
     } else {
-        hipLaunchKernelGGL(k_qkv_rope<false>, grid, dim3(256), 0, s, Wqkv, scales, gamma, x, params,
-            q, kcache_layer, vcache_layer, capacity);
+        LH_QKV(K_FP8, false);
     }
+#undef LH_QKV
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -903,18 +998,23 @@ extern "C" int lh_launch_qkv_attention(int lookup, const uint8_t* Wqkv, float sq
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-extern "C" int lh_launch_gateup_silu(int lookup, const uint8_t* Wgate, const uint8_t* Wup,
+extern "C" int lh_launch_gateup_silu(int strategy, const void* Wgate, const void* Wup,
     float sg, float su, const float* gamma, const float* x, uint32_t count, float* gated,
     hipStream_t s)
 {
     static_assert(LH_INNER % (4 * GATEUP_ROWS) == 0, "gate/up rows per workgroup");
     dim3 grid(LH_INNER / (4 * GATEUP_ROWS), count);
     float2 scales = make_float2(sg, su);
-    if (lookup) {
-        hipLaunchKernelGGL(k_gateup_silu<true>, grid, dim3(512), 0, s, Wgate, Wup, scales, gamma, x, gated);
+#define LH_GATEUP(K, L) hipLaunchKernelGGL((k_gateup_silu<K, L>), grid, dim3(512), 0, s, Wgate, \
+        Wup, scales, gamma, x, gated)
+    if (strategy == LH_ROWS_F32) {
+        LH_GATEUP(K_F32, false);
+    } else if (strategy == LH_ROWS_FP8_LOOKUP) {
+        LH_GATEUP(K_FP8, true);
     } else {
-        hipLaunchKernelGGL(k_gateup_silu<false>, grid, dim3(512), 0, s, Wgate, Wup, scales, gamma, x, gated);
+        LH_GATEUP(K_FP8, false);
     }
+#undef LH_GATEUP
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
