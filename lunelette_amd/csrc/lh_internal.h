@@ -78,6 +78,21 @@ int lh_launch_attention_mfma(const float *q, const float *kcache_layer, const fl
     const lh_step_params *params, uint32_t length, uint32_t count, uint32_t capacity, float *PM,
     float *PT, float *PA, float *out, uint16_t *xs, uint32_t xs_tokens, float *xs_scale,
     hipStream_t s);
+/* Matrix-core projections of at most 32 tokens (mfma_small.hip); xs: activation
+ * planes of `stride` tokens (whole 16-token tiles). qkv: three BF16 planes, RoPE and KV append.
+ * o: two FP16 planes scaled per (token, kv head), x += . gateup: two FP16
+ * planes scaled per token; SiLU(gate)*up as three BF16 planes, which down
+ * takes, x += . */
+int lh_launch_small_qkv(const uint8_t *W, float sq, float sk, float sv, const uint16_t *xs,
+    uint32_t stride, const lh_step_params *params, uint32_t count, float *q, float *kcache_layer,
+    float *vcache_layer, uint32_t capacity, hipStream_t s);
+int lh_launch_small_o(const uint8_t *W, float scale, const uint16_t *xs, uint32_t stride,
+    const float *head_scale, uint32_t count, float *x, hipStream_t s);
+int lh_launch_small_gateup(const uint8_t *Wgate, const uint8_t *Wup, float sg, float su,
+    const uint16_t *xs, uint32_t stride, const float *row_scale, uint32_t count,
+    uint16_t *planes, hipStream_t s);
+int lh_launch_small_down(const uint8_t *W, float scale, const uint16_t *xs, uint32_t stride,
+    uint32_t count, float *x, hipStream_t s);
 /* Block-grid width of the attention kernel. */
 uint32_t lh_attention_blocks(uint32_t length, uint32_t count);
 int lh_launch_embed(const uint16_t *E, const lh_step_params *params, uint32_t count, float *x,

@@ -49,6 +49,7 @@
 #include "lh_device.h"
 #include "lh_internal.h"
 #include "lh_layer.h"
+#include "lh_mfma.h"
 
 #include <stdlib.h>
 
@@ -57,20 +58,11 @@
 
 namespace lh {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 constexpr uint32_t GM = 64;               // tokens per workgroup tile
 constexpr uint32_t GN = 256;              // weight rows per workgroup tile (4 waves x 64)
 constexpr uint32_t BK = 64;               // columns per pipeline stage
 constexpr uint32_t SPLIT_ROWS = 128;      // token stride granule of the split planes
 constexpr uint32_t MAX_N = 2 * LH_INNER;  // widest GEMM: gate|up
-
-// Activation plane formats of the GEMM: three exact BF16 planes (hi + mid + lo),
-// or two FP16 planes of a row scaled by 2^e (h + l, about 22 significant bits).
-enum { PLANES_BF16 = 3, PLANES_F16 = 2 };
 
 __device__ __forceinline__ float4 scale4(float4 v, float s)
 {
@@ -361,39 +353,6 @@ k_qkv_epilogue(const float* __restrict__ partial, size_t split_stride, float3 sc
         *reinterpret_cast<float4*>(kcache + lh_k_index(capacity, 0, head - 32, position, i0 + 64)) =
             out_hi;
     }
-}
-
-// FP8 -> BF16 (or FP16) weight fragments, exact either way: the 16 codes of
-// u (row bytes 16g .. 16g+15 of the step) give the two 8-column k-slices
-// h = 0 (bytes 0..7) and h = 1.
-__device__ __forceinline__ void fp8x16_to_bf16x8x2(u32x4 u, bf16x8& lo, bf16x8& hi)
-{
-    u32x4 a, b;
-    a.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, 1.0f, false));
-    a.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, 1.0f, true));
-    a.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, 1.0f, false));
-    a.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, 1.0f, true));
-    b.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.z, 1.0f, false));
-    b.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.z, 1.0f, true));
-    b.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.w, 1.0f, false));
-    b.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.w, 1.0f, true));
-    lo = __builtin_bit_cast(bf16x8, a);
-    hi = __builtin_bit_cast(bf16x8, b);
-}
-
-__device__ __forceinline__ void fp8x16_to_f16x8x2(u32x4 u, f16x8& lo, f16x8& hi)
-{
-    u32x4 a, b;
-    a.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u.x, 1.0f, false));
-    a.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u.x, 1.0f, true));
-    a.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u.y, 1.0f, false));
-    a.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u.y, 1.0f, true));
-    b.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u.z, 1.0f, false));
-    b.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u.z, 1.0f, true));
-    b.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u.w, 1.0f, false));
-    b.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u.w, 1.0f, true));
-    lo = __builtin_bit_cast(f16x8, a);
-    hi = __builtin_bit_cast(f16x8, b);
 }
 
 // One 64-column stage of a wave's 64 tokens x 16 NF weight rows: A fragments
@@ -1127,6 +1086,40 @@ extern "C" int lh_fp8_gemm(lh_workspace* ws, const uint8_t* d_w, float scale, co
     return combine(ws->d_gemm, splits, (uint32_t)rows, n, B, scale, d_y, 0, s);
 }
 
+// A layer over at most SMALL_TOKENS tokens (mfma_small.hip): no partials; the
+// down input travels as three exact BF16 planes, since its workgroups see too few
+// columns for a scale. The planes are SMALL_TOKENS tall; the down input's
+// follow the other inputs'. (2 tokens 87 -> 59 us, 16 91 -> 63, 17 92 -> 77, 32
+// 100 -> 86: three tiles would lose to the 64-token tiles' 103.)
+constexpr uint32_t SMALL_TOKENS = 32;
+
+static int layer_small(const lh_layer_weights* w, float* d_x, float* d_keys, float* d_values,
+    lh_workspace* ws, int input_split, const float* next_norm, hipStream_t s)
+{
+    const uint32_t n = (uint32_t)ws->count, C = (uint32_t)ws->capacity, T = SMALL_TOKENS;
+    uint16_t* xs = ws->d_split;
+    uint16_t* xd = xs + 3 * T * LH_QUERY;
+    float* scale_a = token_scales(ws);
+    float* scale_b = group_scales(ws);
+    if ((!input_split &&
+            residual_norm_split(NULL, 0, T, 1.0f, d_x, w->input_norm, xs, NULL, n, s)) ||
+        lh_launch_small_qkv(w->qkv, w->scale[0], w->scale[1], w->scale[2], xs, T, ws->d_params, n,
+            ws->d_q, d_keys, d_values, C, s) ||
+        launched_ok("qkv") ||
+        lh_launch_attention_mfma(ws->d_q, d_keys, d_values, ws->d_params, (uint32_t)ws->length,
+            n, C, ws->d_PM, ws->d_PT, ws->d_PA, ws->d_attn, xs, T, scale_b, s) ||
+        launched_ok("attention") ||
+        lh_launch_small_o(w->o, w->scale[3], xs, T, scale_b, n, d_x, s) || launched_ok("o") ||
+        residual_norm_split(NULL, 0, T, 1.0f, d_x, w->post_norm, xs, scale_a, n, s) ||
+        lh_launch_small_gateup(w->gate, w->up, w->scale[4], w->scale[5], xs, T, scale_a, n, xd,
+            s) ||
+        launched_ok("gate/up") ||
+        lh_launch_small_down(w->down, w->scale[6], xd, T, n, d_x, s) || launched_ok("down")) {
+        return -1;
+    }
+    return next_norm ? residual_norm_split(NULL, 0, T, 1.0f, d_x, next_norm, xs, NULL, n, s) : 0;
+}
+
 // One layer over ws->count tokens. input_split: ws->d_split already holds the
 // BF16 planes of input_norm(x) (the previous layer's last kernel wrote them);
 // next_norm: the last kernel also writes them for the following layer (NULL:
@@ -1146,6 +1139,9 @@ extern "C" int lh_layer_forward_mfma(const lh_layer_weights* w, float* d_x, floa
     }
     if (lh_mfma_prepare(ws)) {
         return -1;
+    }
+    if (ws->count <= SMALL_TOKENS) {
+        return layer_small(w, d_x, d_keys, d_values, ws, input_split, next_norm, s);
     }
     const uint32_t n = (uint32_t)ws->count, C = (uint32_t)ws->capacity;
     const uint32_t B = padded_block(ws);

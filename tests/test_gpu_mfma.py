@@ -109,6 +109,30 @@ def test_mfma_layer_small_odd_block(gpu, length, count):
     assert np.max(np.abs(gx - wx) / np.max(np.abs(wx), axis=1, keepdims=True)) < 1e-3
 
 
+@pytest.mark.parametrize("length,count,shift", [(100, 1, 0), (0, 2, 0), (1203, 8, 0), (63, 9, 14),
+                                                (500, 16, 0), (64, 17, -14), (40, 24, 0),
+                                                (3000, 25, 0), (1000, 32, 0), (31, 33, 0)])
+def test_mfma_layer_up_to_32_tokens(gpu, length, count, shift):
+    """The short-message projections (one or two 16-token tiles, half-empty
+    tiles, the first count past them), with gate and up scales times 2^shift:
+    SiLU(gate)*up up to about 1e13 or below about 1e-4. Within the matrix-core
+    layer tolerance of the oracle."""
+    from test_gpu_layer import oracle_layer, run_layer
+    host = dict(syn.layer(SEED, 2))
+    for name in ("scale_gate", "scale_up"):
+        host[name] = math.ldexp(host[name], shift)   # exact: still BF16-exact and normal
+    x = syn.normal_f32(SEED, 9401, count * 3072)
+    kpm = syn.normal_f32(SEED, 9402, length * 1024).reshape(length, 1024)
+    vpm = syn.normal_f32(SEED, 9403, length * 1024).reshape(length, 1024)
+    got = run_layer(gpu, host, x, kpm, vpm, length, count, 4352, lh.PATH_MFMA)
+    want = oracle_layer(host, x, kpm, vpm, length, count, 4352, MIRROR)
+    gx, wx = got[0].reshape(count, 3072), want[0].reshape(count, 3072)
+    assert np.max(np.abs(gx - wx) / np.max(np.abs(wx), axis=1, keepdims=True)) < 1e-3
+    assert np.median(np.abs(gx - wx) / np.maximum(np.abs(wx), 1e-30)) < 1e-5
+    for g, w_ in zip(got[1:], want[1:]):
+        assert np.max(np.abs(g - w_) / np.max(np.abs(w_), axis=1, keepdims=True)) < 1e-5
+
+
 @pytest.mark.parametrize("prompt", [64, 200])
 def test_runtime_mps_prefill_then_decode(gpu, prompt):
     """Chained layers (each layer's last kernel splits the next layer's
