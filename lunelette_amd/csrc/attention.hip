@@ -391,7 +391,9 @@ extern "C" int lh_launch_embed(const uint16_t* E, const lh_step_params* params, 
 // staging and two barriers per block dominated, as here.
 namespace lh {
 
-constexpr uint32_t FA_TQ = 16;                      // tokens per workgroup
+constexpr uint32_t FA_TQ = 16;                      // tokens per subtile
+constexpr int FA_PASSES = 2;                        // subtiles per workgroup
+constexpr uint32_t FA_WG = FA_PASSES * FA_TQ;       // tokens per workgroup
 // Scores in the base-2 domain: s = q.k * (1/sqrt(128)) * log2(e), so the
 // softmax weights are exp2(s - m) on the hardware v_exp_f32; the row maxima
 // in PM are in this domain too (k_attn_merge).
@@ -435,7 +437,7 @@ struct FaCoords {
 __device__ __forceinline__ FaCoords fa_coords(uint32_t tiles)
 {
     const uint32_t w = blockIdx.x, qq = w >> 3;
-    return {(qq % tiles) * FA_TQ, w & 7u, qq / tiles, gridDim.x / (8 * tiles)};
+    return {(qq % tiles) * FA_WG, w & 7u, qq / tiles, gridDim.x / (8 * tiles)};
 }
 
 
@@ -480,28 +482,138 @@ __device__ __forceinline__ uint32_t fb_v_at(uint32_t d, uint32_t r)
     return d * FB_ROW + r * 2;
 }
 
-__device__ __forceinline__ uint32_t fb_hi(float x)
-{
-    return __float_as_uint(x) >> 16;
-}
-
-// Two FP16 planes of four values scaled by f (h = f16(v f), l = f16(v f - h)),
-// packed as two 32-bit pairs each.
+// Two FP16 planes of four values scaled by a power of two f (h = f16(v f), l =
+// f16(v f - h)), packed as two 32-bit pairs each. v f is exact, so the remainder
+// is one fused multiply-add from v.
 __device__ __forceinline__ void f16_planes4(float4 v, float f, uint2& h, uint2& l)
 {
-    float r0, r1, r2, r3;
-    const uint32_t a = f16_hi(v.x * f, r0), b = f16_hi(v.y * f, r1);
-    const uint32_t c = f16_hi(v.z * f, r2), d = f16_hi(v.w * f, r3);
-    h = make_uint2(a | (b << 16), c | (d << 16));
-    l = make_uint2(f16_bits(r0) | (f16_bits(r1) << 16), f16_bits(r2) | (f16_bits(r3) << 16));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    const f16x2 a = __builtin_convertvector((f32x2{v.x * f, v.y * f}), f16x2);
+    const f16x2 b = __builtin_convertvector((f32x2{v.z * f, v.w * f}), f16x2);
+    const f32x2 ra = {__builtin_fmaf(v.x, f, -(float)a.x), __builtin_fmaf(v.y, f, -(float)a.y)};
+    const f32x2 rb = {__builtin_fmaf(v.z, f, -(float)b.x), __builtin_fmaf(v.w, f, -(float)b.y)};
+    h = make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
+    l = make_uint2(__builtin_bit_cast(uint32_t, __builtin_convertvector(ra, f16x2)),
+        __builtin_bit_cast(uint32_t, __builtin_convertvector(rb, f16x2)));
 }
 
-// Two truncated BF16 planes of x: hi and mid (x - hi, truncated).
-__device__ __forceinline__ void fb_split2(float x, uint32_t& h, uint32_t& m)
+// S^T tiles j = 0..3 of NP passes (16-token subtiles): rows positions
+// 16j + 4g + r, columns tokens l16 (A operand K: row 16j + l16, dims 32kc + 8g ..
+// +7, read once for all passes). The fragments of the next group are read
+// while a group's products run, and consecutive products go to four different
+// accumulators: read just in time, with the three products of an accumulator
+// back to back, the waits for LDS and for the previous product took longer than
+// the products.
+__device__ __forceinline__ void fa_lds_wait()
 {
-    const uint32_t hb = __float_as_uint(x) & 0xffff0000u;
-    h = hb >> 16;
-    m = __float_as_uint(x - __uint_as_float(hb)) >> 16;
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0); the next block's loads stay in flight
+}
+
+template <int NP>
+__device__ __forceinline__ void fa_scores(const uint8_t* Kp, uint32_t l16, uint32_t g,
+    const fa_f16x8 (&qh)[NP][4], const fa_f16x8 (&ql)[NP][4], fa_floatx4 (&s)[NP][4])
+{
+    constexpr int W = 4 / NP, GROUPS = 16 / W;   // tiles per group
+    fa_f16x8 kh[2][W], kl[2][W];
+    auto read = [&](int n) {
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const uint32_t at = fb_k_at(16 * (n * W % 4 + w) + l16, 32 * (n * W / 4) + 8 * g);
+            kh[n & 1][w] = *reinterpret_cast<const fa_f16x8*>(Kp + at);
+            kl[n & 1][w] = *reinterpret_cast<const fa_f16x8*>(Kp + FB_KPLANE + at);
+        }
+    };
+#pragma unroll
+    for (int ps = 0; ps < NP; ps++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            s[ps][j] = fa_floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    read(0);
+#pragma unroll
+    for (int n = 0; n < GROUPS; n++) {
+        const int kc = n * W / 4, j0 = n * W % 4;
+        fa_lds_wait();
+        if (n + 1 < GROUPS) {
+            read(n + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int product = 0; product < 3; product++) {
+#pragma unroll
+            for (int w = 0; w < W; w++) {
+#pragma unroll
+                for (int ps = 0; ps < NP; ps++) {
+                    s[ps][j0 + w] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        product == 0 ? kl[n & 1][w] : kh[n & 1][w],
+                        product == 1 ? ql[ps][kc] : qh[ps][kc], s[ps][j0 + w], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// O^T += V^T P^T: A operand of dim tile i: lane (dim 16 i + l16, group g) holds
+// V at positions 32 pc + 4g .. +3 and 32 pc + 16 + 4g .. +3 (two 8-byte reads
+// per plane, read once for all passes), the slots of P^T. Groups and order as
+// in fa_scores.
+template <int NP>
+__device__ __forceinline__ void fa_values(const uint8_t* Vp, uint32_t l16, uint32_t g,
+    const fa_bf16x8 (&ph)[NP][2], const fa_bf16x8 (&pm)[NP][2], fa_floatx4 (&o)[NP][8])
+{
+    constexpr int W = 4 / NP, GROUPS = 16 / W;   // dim tiles per group
+    fa_bf16x8 vh[2][W], vm[2][W];
+    auto read = [&](int n) {
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const uint32_t d = 16 * (n / 2 * W + w) + l16, pc = n % 2;
+            const uint32_t a0 = fb_v_at(d, 32 * pc + 4 * g);
+            const uint32_t a1 = fb_v_at(d, 32 * pc + 16 + 4 * g);
+            const uint2 h0 = *reinterpret_cast<const uint2*>(Vp + a0);
+            const uint2 h1 = *reinterpret_cast<const uint2*>(Vp + a1);
+            const uint2 m0 = *reinterpret_cast<const uint2*>(Vp + FB_VPLANE + a0);
+            const uint2 m1 = *reinterpret_cast<const uint2*>(Vp + FB_VPLANE + a1);
+            vh[n & 1][w] = __builtin_bit_cast(fa_bf16x8, fa_u32x4{h0.x, h0.y, h1.x, h1.y});
+            vm[n & 1][w] = __builtin_bit_cast(fa_bf16x8, fa_u32x4{m0.x, m0.y, m1.x, m1.y});
+        }
+    };
+    read(0);
+#pragma unroll
+    for (int n = 0; n < GROUPS; n++) {
+        const int pc = n % 2, i0 = n / 2 * W;
+        fa_lds_wait();
+        if (n + 1 < GROUPS) {
+            read(n + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int product = 0; product < 3; product++) {
+#pragma unroll
+            for (int w = 0; w < W; w++) {
+#pragma unroll
+                for (int ps = 0; ps < NP; ps++) {
+                    o[ps][i0 + w] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        product == 0 ? vm[n & 1][w] : vh[n & 1][w],
+                        product == 1 ? pm[ps][pc] : ph[ps][pc], o[ps][i0 + w], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// Pairs of values as the packed upper halves of (a, b), and of their remainders.
+__device__ __forceinline__ uint32_t fb_pack(float a, float b)
+{
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+
+__device__ __forceinline__ float fb_rest(float x)
+{
+    return x - __uint_as_float(__float_as_uint(x) & 0xffff0000u);
 }
 
 __global__ void __launch_bounds__(512, 1)
@@ -513,9 +625,9 @@ k_attn_mfma(const float* __restrict__ q, const float* __restrict__ kcache,
     __shared__ __attribute__((aligned(16))) uint8_t Kp[2 * FB_KPLANE];
     __shared__ __attribute__((aligned(16))) uint8_t Vp[2 * FB_VPLANE];
     __shared__ float sk[LH_ATTN_BLOCK];
-    const FaCoords fc = fa_coords((count + 2 * FA_TQ - 1) / (2 * FA_TQ));
+    const FaCoords fc = fa_coords((count + FA_WG - 1) / FA_WG);
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t t0 = 2 * fc.t0 + FA_TQ * (wave >> 2), kvh = fc.kvh;
+    const uint32_t t0 = fc.t0 + FA_TQ * (wave >> 2), kvh = fc.kvh;
     const uint32_t g = lane >> 4, l16 = lane & 15;
     const uint32_t head = kvh * 4 + (wave & 3);
     // The second 16-token subtile can lie past count: it then runs on the
@@ -528,7 +640,7 @@ k_attn_mfma(const float* __restrict__ q, const float* __restrict__ kcache,
     // 2^-eq * log2(e) / sqrt(128) for the lane's token, whose S^T column the
     // lane also holds.
     const uint32_t tq = t0 + l16 <= last ? t0 + l16 : last;
-    fa_f16x8 qh[4], ql[4];
+    fa_f16x8 qh[1][4], ql[1][4];
     float fq;
     {
         const float4* src = reinterpret_cast<const float4*>(
@@ -552,23 +664,24 @@ k_attn_mfma(const float* __restrict__ q, const float* __restrict__ kcache,
             uint2 h0, l0, h1, l1;
             f16_planes4(a[kc], f, h0, l0);
             f16_planes4(b[kc], f, h1, l1);
-            qh[kc] = __builtin_bit_cast(fa_f16x8, fa_u32x4{h0.x, h0.y, h1.x, h1.y});
-            ql[kc] = __builtin_bit_cast(fa_f16x8, fa_u32x4{l0.x, l0.y, l1.x, l1.y});
+            qh[0][kc] = __builtin_bit_cast(fa_f16x8, fa_u32x4{h0.x, h0.y, h1.x, h1.y});
+            ql[0][kc] = __builtin_bit_cast(fa_f16x8, fa_u32x4{l0.x, l0.y, l1.x, l1.y});
         }
     }
     const uint32_t limit = length + tq;   // the lane's token's last visible position
     // Online-softmax state of the lane's token (replicated over its four
     // lane groups) and O^T tiles i: dims 16 i + 4g + r of the lane's token.
     float m = -__builtin_inff(), l = 0.0f;
-    fa_floatx4 o[8];
+    fa_floatx4 ot[1][8];
+    fa_floatx4 (&o)[8] = ot[0];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         o[i] = fa_floatx4{0.f, 0.f, 0.f, 0.f};
     }
     // The block range and the staging's visible rows follow the workgroup's
     // last token (both subtiles share every barrier and every staged block).
-    const uint32_t tw = 2 * fc.t0;
-    const uint32_t last_wg = (tw + 2 * FA_TQ < count ? tw + 2 * FA_TQ : count) - 1;
+    const uint32_t tw = fc.t0;
+    const uint32_t last_wg = (tw + FA_WG < count ? tw + FA_WG : count) - 1;
     const uint32_t nb = (length + last_wg + 1 + LH_ATTN_BLOCK - 1) / LH_ATTN_BLOCK;
     const uint32_t splits = fc.splits, z = fc.z;
     const uint32_t per = (nb + splits - 1) / splits;
@@ -663,42 +776,23 @@ k_attn_mfma(const float* __restrict__ q, const float* __restrict__ kcache,
             v_item(j, d, r0);
             const float v0 = b * LH_ATTN_BLOCK + r0 <= visible ? vr[2 * j] : 0.0f;
             const float v1 = b * LH_ATTN_BLOCK + r0 + 1 <= visible ? vr[2 * j + 1] : 0.0f;
-            uint32_t h0, m0, h1, m1;
-            fb_split2(v0, h0, m0);
-            fb_split2(v1, h1, m1);
             const uint32_t at = fb_v_at(d, r0);
-            *reinterpret_cast<uint32_t*>(Vp + at) = h0 | (h1 << 16);
-            *reinterpret_cast<uint32_t*>(Vp + FB_VPLANE + at) = m0 | (m1 << 16);
+            *reinterpret_cast<uint32_t*>(Vp + at) = fb_pack(v0, v1);
+            *reinterpret_cast<uint32_t*>(Vp + FB_VPLANE + at) = fb_pack(fb_rest(v0), fb_rest(v1));
         }
         __syncthreads();
         if (b + 1 < b_end) {
             load_block(b + 1);   // in flight during this block's MFMAs
         }
-        // S^T tiles j = 0..3: rows positions 16j + 4g + r, columns tokens l16
-        // (A operand K: row 16j + l16, dims 32kc + 8g .. +7).
-        fa_floatx4 s[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            s[j] = zero;
-        }
-#pragma unroll
-        for (int kc = 0; kc < 4; kc++) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t at = fb_k_at(16 * j + l16, 32 * kc + 8 * g);
-                const fa_f16x8 kh = *reinterpret_cast<const fa_f16x8*>(Kp + at);
-                const fa_f16x8 kl = *reinterpret_cast<const fa_f16x8*>(Kp + FB_KPLANE + at);
-                s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[kc], s[j], 0, 0, 0);
-                s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[kc], s[j], 0, 0, 0);
-                s[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[kc], s[j], 0, 0, 0);
-            }
-        }
+        fa_floatx4 st[1][4];
+        fa_scores<1>(Kp, l16, g, qh, ql, st);
+        const fa_floatx4 (&s)[4] = st[0];
         // Scale (2^-ek of the row's position, fq of the token), causal mask,
         // online softmax of the lane's token over its 16 values and its three
         // other lane groups; P^T as the PV B operand of position chunk pc:
         // k slots 0..3 = positions 32 pc + 4g + r (tile j = 2 pc), slots 4..7
         // = 32 pc + 16 + 4g + r (tile j = 2 pc + 1).
-        fa_bf16x8 ph[2], pm[2];
+        fa_bf16x8 ph[1][2], pm[1][2];
         {
             float v[16];
             float mx = -__builtin_inff();
@@ -729,14 +823,11 @@ k_attn_mfma(const float* __restrict__ q, const float* __restrict__ kcache,
                     const float e1 = empty ? 0.0f : __builtin_amdgcn_exp2f(v[8 * pc + k + 1] - m_new);
                     sum = sum + e0;
                     sum = sum + e1;
-                    uint32_t h0, m0, h1, m1;
-                    fb_split2(e0, h0, m0);
-                    fb_split2(e1, h1, m1);
-                    hi[k / 2] = h0 | (h1 << 16);
-                    mid[k / 2] = m0 | (m1 << 16);
+                    hi[k / 2] = fb_pack(e0, e1);
+                    mid[k / 2] = fb_pack(fb_rest(e0), fb_rest(e1));
                 }
-                ph[pc] = __builtin_bit_cast(fa_bf16x8, hi);
-                pm[pc] = __builtin_bit_cast(fa_bf16x8, mid);
+                ph[0][pc] = __builtin_bit_cast(fa_bf16x8, hi);
+                pm[0][pc] = __builtin_bit_cast(fa_bf16x8, mid);
             }
             l = l * alpha + col4_sum(sum);
             m = m_new;
@@ -745,27 +836,7 @@ k_attn_mfma(const float* __restrict__ q, const float* __restrict__ kcache,
                 o[i] = o[i] * alpha;
             }
         }
-        // O^T += V^T P^T: A operand of dim tile i: lane (dim 16 i + l16, group
-        // g) holds V at positions 32 pc + 4g .. +3 and 32 pc + 16 + 4g .. +3
-        // (two 8-byte reads per plane), the slots of P^T above.
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const uint32_t d = 16 * i + l16;
-#pragma unroll
-            for (int pc = 0; pc < 2; pc++) {
-                const uint32_t a0 = fb_v_at(d, 32 * pc + 4 * g);
-                const uint32_t a1 = fb_v_at(d, 32 * pc + 16 + 4 * g);
-                const uint2 h0 = *reinterpret_cast<const uint2*>(Vp + a0);
-                const uint2 h1 = *reinterpret_cast<const uint2*>(Vp + a1);
-                const uint2 m0 = *reinterpret_cast<const uint2*>(Vp + FB_VPLANE + a0);
-                const uint2 m1 = *reinterpret_cast<const uint2*>(Vp + FB_VPLANE + a1);
-                const fa_bf16x8 vh = __builtin_bit_cast(fa_bf16x8, fa_u32x4{h0.x, h0.y, h1.x, h1.y});
-                const fa_bf16x8 vm = __builtin_bit_cast(fa_bf16x8, fa_u32x4{m0.x, m0.y, m1.x, m1.y});
-                o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vm, ph[pc], o[i], 0, 0, 0);
-                o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, pm[pc], o[i], 0, 0, 0);
-                o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, ph[pc], o[i], 0, 0, 0);
-            }
-        }
+        fa_values<1>(Vp, l16, g, ph, pm, ot);
     }
     // Output planes (one split): each token's four query heads of this kv
     // head (512 columns, one K split of the o projection) share one power of
@@ -830,65 +901,69 @@ k_attn_mfma(const float* __restrict__ q, const float* __restrict__ kcache,
     }
 }
 
-// The wide variant for long prefixes (k_attn_mfma_wide): 64-token
-// workgroups, each wave running two 16-token subtiles over every staged
-// block, so each block is split into planes once per 64 tokens. The two
-// passes' Q planes and O accumulators double the per-wave state; the raw
-// K/V tiles therefore come to LDS by direct loads (136 KiB of LDS) instead of
-// through registers, and each K and V fragment read from LDS feeds both
-// passes. Measured (attention + merge, 256 tokens): 88.5 against 95.8 us
-// after a 4096-token prefix, 148 against 170 us after 8192, 255 against 304
-// us after 16128; slower on short prefixes (28.6 against 22.5 us with no
-// prefix: half the workgroups) and for 64 tokens, where the launcher keeps
-// k_attn_mfma.
-constexpr uint32_t WIDE_PASSES = 2;                          // subtiles per wave
-constexpr uint32_t WIDE_WG = 2 * WIDE_PASSES * FA_TQ;        // tokens per workgroup
-constexpr uint32_t WIDE_MIN_LENGTH = 2048;                   // prefix from which it pays
-constexpr uint32_t WIDE_MIN_COUNT = 128;                     // tokens from which it pays
+// The variant for long prefixes: the same 32 tokens in four waves, wave w query
+// head 4 kvh + w over both 16-token subtiles, two workgroups per CU. Each K and V
+// fragment read from LDS feeds two products, a workgroup's loads, staging,
+// softmax and products overlap the other's, and V is staged behind the softmax,
+// so that both tiles' loads have half a block's time to land (K's during P.V,
+// V's during the scores). Blocks wholly before the tile skip the causal mask,
+// and blocks that raise no maximum the rescaling of O.
+// Measured (kernel trace), k_attn_mfma and the former 64-token variant before:
+// 64 tokens after 15872 positions 86 -> 70 us (and 3 us more in the merge of
+// twice as many splits), 256 after 4096 80 -> 77 us; the layer of 130 tokens after
+// 5000 231 -> 214 us; with one workgroup per CU 80 and 88 us. After short prefixes its 4-wave workgroups lose (201 tokens after 256:
+// 19.2 against 17.9 us).
+constexpr uint32_t FA_LONG_LENGTH = 2048;   // prefix from which it pays
 
-__global__ void __launch_bounds__(512, 1)
-k_attn_mfma_wide(const float* __restrict__ q, const float* __restrict__ kcache,
+// The thread id again, where a value held for it across the block loop would
+// spill.
+__device__ __forceinline__ uint32_t fa_thread()
+{
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
+__global__ void __launch_bounds__(256, 2)
+k_attn_mfma_long(const float* __restrict__ q, const float* __restrict__ kcache,
     const float* __restrict__ vcache, uint32_t length, uint32_t count, uint32_t capacity,
     float* __restrict__ PM, float* __restrict__ PT, float* __restrict__ PA, float* __restrict__ out,
     uint16_t* __restrict__ xs, uint32_t xs_tokens, float* __restrict__ xs_scale)
 {
+    constexpr int NP = FA_PASSES;
     __shared__ __attribute__((aligned(16))) uint8_t Kp[2 * FB_KPLANE];
     __shared__ __attribute__((aligned(16))) uint8_t Vp[2 * FB_VPLANE];
     __shared__ float sk[LH_ATTN_BLOCK];
-    const FaCoords fc = fa_coords((count + WIDE_WG - 1) / WIDE_WG);
-    const uint32_t tid = threadIdx.x, kvh = fc.kvh;
-    uint32_t lane = tid & 63, wave = tid >> 6;
-    uint32_t g = lane >> 4, l16 = lane & 15;
-    uint32_t head = kvh * 4 + (wave & 3);
-    // The workgroup's WIDE_WG tokens start at tw; wave w runs 16-token subtiles
-    // 2 pass + w / 4 in passes 0 and 1 over every staged block.
-    const uint32_t tw = fc.t0 * (WIDE_WG / FA_TQ);
-    const uint32_t last_wg = (tw + WIDE_WG < count ? tw + WIDE_WG : count) - 1;
-    // A subtile can lie past count: it then runs on the last real subtile's
-    // tokens (clamped) and stores nothing.
-    const uint32_t last_sub = (count - 1) / FA_TQ * FA_TQ;
-    uint32_t t0[WIDE_PASSES], last[WIDE_PASSES];
-    // The lane's token in pass ps (clamped to the subtile's last real token).
-    auto tq_of = [&](int ps) { return t0[ps] + l16 <= last[ps] ? t0[ps] + l16 : last[ps]; };
+    __shared__ float gmax[FA_WG][4];
+    const FaCoords fc = fa_coords((count + FA_WG - 1) / FA_WG);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, kvh = fc.kvh;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t g = lane >> 4, l16 = lane & 15;
+    const uint32_t head = kvh * 4 + wave;
+    // The workgroup's tokens start at tw; pass ps runs the 16 tokens from
+    // tw + 16 ps. A subtile past count repeats the last token and stores nothing.
+    const uint32_t tw = fc.t0;
+    const uint32_t last_wg = (tw + FA_WG < count ? tw + FA_WG : count) - 1;
+    // The lane's token in pass ps (clamped to the last real token).
+    auto token = [&](int ps) {
+        const uint32_t t = tw + FA_TQ * ps + l16;
+        return t < count ? t : count - 1;
+    };
     // Q operand of k-chunk kc (the B operand of S^T = K Q^T): lane (token
     // l16, group g) holds dims 32 kc + 8g .. +7, as two FP16 planes of the
     // row scaled by 2^eq (its largest magnitude into [2^14, 2^15)). fq =
     // 2^-eq * log2(e) / sqrt(128) for the lane's token, whose S^T column the
     // lane also holds.
-    fa_f16x8 qh[WIDE_PASSES][4], ql[WIDE_PASSES][4];
-    float fq[WIDE_PASSES];
+    fa_f16x8 qh[NP][4], ql[NP][4];
+    float fq[NP];
     // Online-softmax state of the lane's token (replicated over its four
     // lane groups) and O^T tiles i: dims 16 i + 4g + r of the lane's token.
-    float m[WIDE_PASSES], l[WIDE_PASSES];
-    fa_floatx4 o[WIDE_PASSES][8];
+    float m[NP], l[NP];
+    fa_floatx4 o[NP][8];
 #pragma unroll
-    for (int ps = 0; ps < WIDE_PASSES; ps++) {
-        t0[ps] = tw + FA_TQ * (2 * ps + (wave >> 2));
-        const uint32_t t0c = t0[ps] < count ? t0[ps] : last_sub;
-        last[ps] = (t0c + FA_TQ < count ? t0c + FA_TQ : count) - 1;   // last real token
-        const uint32_t tq = t0[ps] + l16 <= last[ps] ? t0[ps] + l16 : last[ps];
+    for (int ps = 0; ps < NP; ps++) {
         const float4* src = reinterpret_cast<const float4*>(
-            q + (size_t)tq * LH_QUERY + head * LH_HEAD_DIM + 8 * g);
+            q + (size_t)token(ps) * LH_QUERY + head * LH_HEAD_DIM + 8 * g);
         float4 a[4], b[4];
         float mx = 0.0f;
 #pragma unroll
@@ -919,75 +994,71 @@ k_attn_mfma_wide(const float* __restrict__ q, const float* __restrict__ kcache,
         }
     }
     // The block range and the staging's visible rows follow the workgroup's
-    // last token (all subtiles share every barrier and every staged block).
+    // last token.
     const uint32_t nb = (length + last_wg + 1 + LH_ATTN_BLOCK - 1) / LH_ATTN_BLOCK;
     const uint32_t splits = fc.splits, z = fc.z;
     const uint32_t per = (nb + splits - 1) / splits;
     const uint32_t b_begin = z * per < nb ? z * per : nb;
     const uint32_t b_end = b_begin + per < nb ? b_begin + per : nb;
     const size_t head_base = lh_kv_index(capacity, 0, kvh, 0);
-    // Raw K and V of block b go to LDS by direct loads (the next block's
-    // issued once this block's staging has read them, in flight during its
-    // MFMAs): the tiles as they lie in the cache, K in lh_ktile_word order,
-    // V row-major. Wave w, load i copies the 1 KiB chunk 8i + w of each.
-    // V staging item j (0..7) of thread tid: lane l of wave w takes dim
-    // 16 ((j + l / 16) % 8) + l % 16 and positions r0, r0 + 1 with
-    // r0 = 2 (4 w + l / 16). The four 16-lane groups of a wave read four
-    // different 16-dim blocks of the raw tile, so the reads of the row-major
-    // raw V land on 64 distinct banks (rows are 128 words apart, so without
-    // the rotation the groups' reads met on the same 16 banks); the
-    // packed-pair writes of the transposed planes land on 64 distinct banks
-    // either way (row d starts 36 d words in).
-    auto v_item = [&](int j, uint32_t& d, uint32_t& r0) {
-        d = 16 * ((j + (lane >> 4)) & 7) + (lane & 15);
-        r0 = 2 * (4 * wave + (lane >> 4));
-    };
-    // K: wave w takes positions 8w .. 8w+7 of the block; lane l holds
-    // position kp = 8w + (l % 32) / 4, quarter kq = l % 4, dims
-    // 32 kq + 4 (2i + l / 32) .. +3 for i = 0..3, so the eight lanes of a
-    // position hold all its 128 dims.
-    const uint32_t kp = 8 * wave + ((lane & 31) >> 2), kq = lane & 3, khalf = lane >> 5;
-    __shared__ __attribute__((aligned(16))) fa_floatx4 Kraw[LH_ATTN_BLOCK * LH_HEAD_DIM / 4];
-    __shared__ __attribute__((aligned(16))) fa_floatx4 Vraw[LH_ATTN_BLOCK * LH_HEAD_DIM / 4];
-    auto load_block = [&](uint32_t b) {
+    // K: wave w takes positions 16w .. 16w + 15 of the block; lane l holds
+    // position kp = 16w + l / 4, quarter kq = l % 4: its dims 32 kq + 4i .. +3
+    // for i = 0..7 are the tile's words (8w + i) * 64 + l, and the four lanes of
+    // a quad hold the position's 128 dims.
+    const uint32_t kp = 16 * wave + (lane >> 2), kq = lane & 3;
+    // V: item (jj, j), j < 8: lane l of wave w takes dim 16 j + l % 16 and
+    // positions r0, r0 + 1 with r0 = 2 (4 (w + 4 jj) + l / 16), so one wave
+    // instruction covers 16 dims x 4 position pairs: the loads read 8 x 64
+    // contiguous bytes, and the packed-pair writes of the transposed planes
+    // land on 64 distinct banks.
+    fa_floatx4 kr[8];
+    float vr[32];
+    auto load_k = [&](uint32_t b) {
         const fa_floatx4* kb = reinterpret_cast<const fa_floatx4*>(
-            kcache + head_base + (size_t)b * LH_ATTN_BLOCK * LH_HEAD_DIM);
-        const fa_floatx4* vb = reinterpret_cast<const fa_floatx4*>(
-            vcache + head_base + (size_t)b * LH_ATTN_BLOCK * LH_HEAD_DIM);
+            kcache + head_base + (size_t)b * LH_ATTN_BLOCK * LH_HEAD_DIM) + wave * 512 + lane;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t c = 8 * i + wave;
-            __builtin_amdgcn_global_load_lds(kb + 64 * c + lane, Kraw + 64 * c, 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(vb + 64 * c + lane, Vraw + 64 * c, 16, 0, 0);
+        for (int i = 0; i < 8; i++) {
+            kr[i] = kb[64 * i];
+        }
+    };
+    auto load_v = [&](uint32_t b) {
+        const float* vf = vcache + head_base + (size_t)b * LH_ATTN_BLOCK * LH_HEAD_DIM +
+            2 * (4 * wave + g) * LH_HEAD_DIM + l16;
+#pragma unroll
+        for (int jj = 0; jj < 2; jj++) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                vr[16 * jj + 2 * j] = vf[32 * jj * LH_HEAD_DIM + 16 * j];
+                vr[16 * jj + 2 * j + 1] = vf[(32 * jj + 1) * LH_HEAD_DIM + 16 * j];
+            }
         }
     };
     if (b_begin < b_end) {
-        load_block(b_begin);
+        load_k(b_begin);
     }
     // Rows past the tile's last visible position hold whatever an earlier
     // sequence (or a failed step) left in the cache; they are staged as zeros
     // (0 * Inf would be NaN in P.V).
     const uint32_t visible = length + last_wg;
-    const fa_floatx4 zero = fa_floatx4{0.f, 0.f, 0.f, 0.f};
     for (uint32_t b = b_begin; b < b_end; b++) {
-        // Block b's raw tiles have landed (each wave waits for its own direct
-        // loads) and the previous block's planes are consumed.
-        __builtin_amdgcn_s_waitcnt(0x0f70);
-        __syncthreads();
-        {
-            fa_floatx4 kr[4];
+        const uint32_t first = b * LH_ATTN_BLOCK;
+        const bool ragged = first + LH_ATTN_BLOCK - 1 > visible;
+        if (ragged) {
+            const uint32_t t = fa_thread();
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                kr[i] = Kraw[lh_ktile_word(kp, kq, 2 * i + khalf)];
+            for (int i = 0; i < 8; i++) {
+                kr[i] = (t >> 2) <= visible - first ? kr[i] : fa_floatx4{0.f, 0.f, 0.f, 0.f};
             }
-            // K: the position's largest magnitude over its eight lanes (a
-            // DPP quad, then the other 32-lane half), its power of two 2^ek
-            // (into [2^14, 2^15)), and the two FP16 planes; sk[p] = 2^-ek.
-            const bool kvis = b * LH_ATTN_BLOCK + kp <= visible;
+        }
+        // (The K planes of the block before were consumed before its second
+        // barrier, its V planes are before this block's first.)
+        {
+            // K: the position's largest magnitude over its quad, its power of
+            // two 2^ek (into [2^14, 2^15)), and the two FP16 planes; sk[p] =
+            // 2^-ek.
             float mx = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                kr[i] = kvis ? kr[i] : zero;
+            for (int i = 0; i < 8; i++) {
                 mx = fmaxf(mx, fmaxf(fmaxf(fabsf(kr[i].x), fabsf(kr[i].y)),
                                      fmaxf(fabsf(kr[i].z), fabsf(kr[i].w))));
             }
@@ -995,180 +1066,128 @@ k_attn_mfma_wide(const float* __restrict__ q, const float* __restrict__ kcache,
                 0xf, false)));   // quad_perm [1,0,3,2]
             mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(mx), 0x4E, 0xf,
                 0xf, false)));   // quad_perm [2,3,0,1]
-            const uint32_t mu = __float_as_uint(mx);
-            const auto p32 = __builtin_amdgcn_permlane32_swap(mu, mu, false, false);
-            const int ek = row_exponent(fmaxf(__uint_as_float(p32[0]), __uint_as_float(p32[1])));
-            if ((lane & 35) == 0) {
-                // The position again from the thread id (a register held for
-                // it across the loop would spill).
-                uint32_t t = threadIdx.x;
-                asm volatile("" : "+v"(t));
-                sk[8 * (t >> 6) + ((t & 31) >> 2)] = exp2i(-ek);
+            const int ek = row_exponent(mx);
+            if (kq == 0) {
+                sk[kp] = exp2i(-ek);
             }
             const float f = exp2i(ek);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < 8; i++) {
                 uint2 h, lo;
                 f16_planes4(make_float4(kr[i].x, kr[i].y, kr[i].z, kr[i].w), f, h, lo);
-                const uint32_t at = fb_k_at(kp, 32 * kq + 4 * (2 * i + khalf));
+                const uint32_t at = fb_k_at(kp, 32 * kq + 4 * i);
                 *reinterpret_cast<uint2*>(Kp + at) = h;
                 *reinterpret_cast<uint2*>(Kp + FB_KPLANE + at) = lo;
             }
         }
-        const float* vf = reinterpret_cast<const float*>(Vraw);
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            uint32_t d, r0;
-            v_item(j, d, r0);
-            const float v0 = b * LH_ATTN_BLOCK + r0 <= visible ? vf[r0 * LH_HEAD_DIM + d] : 0.0f;
-            const float v1 = b * LH_ATTN_BLOCK + r0 + 1 <= visible ?
-                vf[(r0 + 1) * LH_HEAD_DIM + d] : 0.0f;
-            uint32_t h0, m0, h1, m1;
-            fb_split2(v0, h0, m0);
-            fb_split2(v1, h1, m1);
-            const uint32_t at = fb_v_at(d, r0);
-            *reinterpret_cast<uint32_t*>(Vp + at) = h0 | (h1 << 16);
-            *reinterpret_cast<uint32_t*>(Vp + FB_VPLANE + at) = m0 | (m1 << 16);
-        }
         __syncthreads();
-        if (b + 1 < b_end) {
-            load_block(b + 1);   // in flight during this block's MFMAs
-        }
-        // S^T tiles j = 0..3 of each pass: rows positions 16j + 4g + r,
-        // columns tokens l16 (A operand K: row 16j + l16, dims 32kc + 8g ..
-        // +7, read once for both passes).
-        fa_floatx4 s[WIDE_PASSES][4];
-#pragma unroll
-        for (int ps = 0; ps < WIDE_PASSES; ps++) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                s[ps][j] = zero;
-            }
-        }
-#pragma unroll
-        for (int kc = 0; kc < 4; kc++) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t at = fb_k_at(16 * j + l16, 32 * kc + 8 * g);
-                const fa_f16x8 kh = *reinterpret_cast<const fa_f16x8*>(Kp + at);
-                const fa_f16x8 kl = *reinterpret_cast<const fa_f16x8*>(Kp + FB_KPLANE + at);
-#pragma unroll
-                for (int ps = 0; ps < WIDE_PASSES; ps++) {
-                    s[ps][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[ps][kc], s[ps][j], 0, 0, 0);
-                    s[ps][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[ps][kc], s[ps][j], 0, 0, 0);
-                    s[ps][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[ps][kc], s[ps][j], 0, 0, 0);
-                }
-            }
-        }
+        load_v(b);   // in flight during the scores and the softmax
+        fa_floatx4 s[NP][4];
+        fa_scores<NP>(Kp, l16, g, qh, ql, s);
         // Scale (2^-ek of the row's position, fq of the token), causal mask,
         // online softmax of the lane's token over its 16 values and its three
         // other lane groups; P^T as the PV B operand of position chunk pc:
         // k slots 0..3 = positions 32 pc + 4g + r (tile j = 2 pc), slots 4..7
         // = 32 pc + 16 + 4g + r (tile j = 2 pc + 1).
-        fa_bf16x8 ph[WIDE_PASSES][2], pm[WIDE_PASSES][2];
+        const bool whole = first + LH_ATTN_BLOCK - 1 <= length + tw;   // for every token
+        fa_bf16x8 ph[NP][2], pm[NP][2];
 #pragma unroll
-        for (int ps = 0; ps < WIDE_PASSES; ps++) {
-            // The scaled, masked scores in place (s[ps] holds them from here).
+        for (int ps = 0; ps < NP; ps++) {
             float mx = -__builtin_inff();
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const fa_floatx4 fk = *reinterpret_cast<const fa_floatx4*>(sk + 16 * j + 4 * g);
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const uint32_t p = b * LH_ATTN_BLOCK + 16 * j + 4 * g + r;
-                    const float x = p <= length + tq_of(ps) ? s[ps][j][r] * fk[r] * fq[ps] :
-                        -__builtin_inff();
-                    s[ps][j][r] = x;
-                    mx = fmaxf(mx, x);
+                    s[ps][j][r] = s[ps][j][r] * fk[r] * fq[ps];
+                }
+            }
+            if (!whole) {
+                const uint32_t t = fa_thread() & 63, tq = tw + FA_TQ * ps + (t & 15);
+                // Positions of the block the token sees, less the lane's first.
+                const int live = (int)(length + (tq < count ? tq : count - 1)) - (int)first -
+                    4 * (int)(t >> 4);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        s[ps][j][r] = 16 * j + r > live ? -__builtin_inff() : s[ps][j][r];
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    mx = fmaxf(mx, s[ps][j][r]);
                 }
             }
             mx = col4_max(mx);
-            // A split can start past a token's last visible position: keep
-            // its row empty (no exp of -inf - -inf).
+            // A split can start past a token's last visible position: its row
+            // stays empty (weights exp2(-inf - 0) = 0, no exp of -inf - -inf).
             const float m_new = fmaxf(m[ps], mx);
             const bool empty = m_new == -__builtin_inff();
             const float alpha = empty ? 1.0f : __builtin_amdgcn_exp2f(m[ps] - m_new);
+            const float base = empty ? 0.0f : m_new;
             float sum = 0.0f;
 #pragma unroll
             for (int pc = 0; pc < 2; pc++) {
                 fa_u32x4 hi, mid;
 #pragma unroll
                 for (int k = 0; k < 8; k += 2) {
-                    const float x0 = s[ps][2 * pc + k / 4][k % 4];
-                    const float x1 = s[ps][2 * pc + (k + 1) / 4][(k + 1) % 4];
-                    const float e0 = empty ? 0.0f : __builtin_amdgcn_exp2f(x0 - m_new);
-                    const float e1 = empty ? 0.0f : __builtin_amdgcn_exp2f(x1 - m_new);
+                    const float e0 = __builtin_amdgcn_exp2f(s[ps][2 * pc + k / 4][k % 4] - base);
+                    const float e1 = __builtin_amdgcn_exp2f(
+                        s[ps][2 * pc + (k + 1) / 4][(k + 1) % 4] - base);
                     sum = sum + e0;
                     sum = sum + e1;
-                    uint32_t h0, m0, h1, m1;
-                    fb_split2(e0, h0, m0);
-                    fb_split2(e1, h1, m1);
-                    hi[k / 2] = h0 | (h1 << 16);
-                    mid[k / 2] = m0 | (m1 << 16);
+                    hi[k / 2] = fb_pack(e0, e1);
+                    mid[k / 2] = fb_pack(fb_rest(e0), fb_rest(e1));
                 }
                 ph[ps][pc] = __builtin_bit_cast(fa_bf16x8, hi);
                 pm[ps][pc] = __builtin_bit_cast(fa_bf16x8, mid);
             }
             l[ps] = l[ps] * alpha + col4_sum(sum);
             m[ps] = m_new;
+            // (A block that raises no row's maximum leaves O as it is.)
+            if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                o[ps][i] = o[ps][i] * alpha;
-            }
-        }
-        // O^T += V^T P^T: A operand of dim tile i: lane (dim 16 i + l16, group
-        // g) holds V at positions 32 pc + 4g .. +3 and 32 pc + 16 + 4g .. +3
-        // (two 8-byte reads per plane, read once for both passes), the slots
-        // of P^T above.
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const uint32_t d = 16 * i + l16;
-#pragma unroll
-            for (int pc = 0; pc < 2; pc++) {
-                const uint32_t a0 = fb_v_at(d, 32 * pc + 4 * g);
-                const uint32_t a1 = fb_v_at(d, 32 * pc + 16 + 4 * g);
-                const uint2 h0 = *reinterpret_cast<const uint2*>(Vp + a0);
-                const uint2 h1 = *reinterpret_cast<const uint2*>(Vp + a1);
-                const uint2 m0 = *reinterpret_cast<const uint2*>(Vp + FB_VPLANE + a0);
-                const uint2 m1 = *reinterpret_cast<const uint2*>(Vp + FB_VPLANE + a1);
-                const fa_bf16x8 vh = __builtin_bit_cast(fa_bf16x8, fa_u32x4{h0.x, h0.y, h1.x, h1.y});
-                const fa_bf16x8 vm = __builtin_bit_cast(fa_bf16x8, fa_u32x4{m0.x, m0.y, m1.x, m1.y});
-#pragma unroll
-                for (int ps = 0; ps < WIDE_PASSES; ps++) {
-                    o[ps][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vm, ph[ps][pc], o[ps][i], 0, 0, 0);
-                    o[ps][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, pm[ps][pc], o[ps][i], 0, 0, 0);
-                    o[ps][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, ph[ps][pc], o[ps][i], 0, 0, 0);
+                for (int i = 0; i < 8; i++) {
+                    o[ps][i] = o[ps][i] * alpha;
                 }
             }
         }
+        if (ragged) {
+            const uint32_t t = 2 * (fa_thread() >> 4);   // r0 of items jj = 0
+#pragma unroll
+            for (int i = 0; i < 32; i++) {
+                vr[i] = t + 32 * (i >> 4) + (i & 1) <= visible - first ? vr[i] : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int jj = 0; jj < 2; jj++) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float v0 = vr[16 * jj + 2 * j], v1 = vr[16 * jj + 2 * j + 1];
+                const uint32_t at = fb_v_at(16 * j + l16, 2 * (4 * (wave + 4 * jj) + g));
+                *reinterpret_cast<uint32_t*>(Vp + at) = fb_pack(v0, v1);
+                *reinterpret_cast<uint32_t*>(Vp + FB_VPLANE + at) = fb_pack(fb_rest(v0),
+                    fb_rest(v1));
+            }
+        }
+        __syncthreads();
+        // The next block's K, in flight during the products (the last block
+        // requests itself).
+        load_k(b + 1 < b_end ? b + 1 : b);
+        fa_values<NP>(Vp, l16, g, ph, pm, o);
     }
     // Output planes (one split): each token's four query heads of this kv
     // head (512 columns, one K split of the o projection) share one power of
     // two 2^e, their largest magnitude into [2^14, 2^15), before the split
     // into two FP16 planes; xs_scale[t][kv head] = 2^-e. The heads' maxima
     // meet in LDS before any wave leaves.
-    // The lane's coordinates again (held across the block loop they would
-    // spill: the loop needs every register).
-    {
-        uint32_t tid_e = threadIdx.x;
-        asm volatile("" : "+v"(tid_e));
-        lane = tid_e & 63;
-        g = lane >> 4;
-        l16 = lane & 15;
-        const uint32_t wave_e = __builtin_amdgcn_readfirstlane(tid_e >> 6);
-#pragma unroll
-        for (int ps = 0; ps < WIDE_PASSES; ps++) {
-            t0[ps] = tw + FA_TQ * (2 * ps + (wave_e >> 2));
-            const uint32_t t0c = t0[ps] < count ? t0[ps] : last_sub;
-            last[ps] = (t0c + FA_TQ < count ? t0c + FA_TQ : count) - 1;
-        }
-        head = kvh * 4 + (wave_e & 3);
-        wave = wave_e;
-    }
-    __shared__ float gmax[WIDE_WG][4];
     if (splits == 1 && xs) {
 #pragma unroll
-        for (int ps = 0; ps < WIDE_PASSES; ps++) {
+        for (int ps = 0; ps < NP; ps++) {
             float mr = 0.0f;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
@@ -1177,7 +1196,7 @@ k_attn_mfma_wide(const float* __restrict__ q, const float* __restrict__ kcache,
             }
             mr = col4_max(mr) / l[ps];
             if (g == 0) {
-                gmax[t0[ps] - tw + l16][wave & 3] = mr;
+                gmax[FA_TQ * ps + l16][wave] = mr;
             }
         }
         __syncthreads();
@@ -1185,17 +1204,17 @@ k_attn_mfma_wide(const float* __restrict__ q, const float* __restrict__ kcache,
     // The lane's token and its O^T values: dims 16 i + 4g .. +3.
     const uint32_t nbc = capacity / LH_ATTN_BLOCK;
 #pragma unroll
-    for (int ps = 0; ps < WIDE_PASSES; ps++) {
-        const uint32_t t = t0[ps] + l16;
-        if (t0[ps] >= count || t > last[ps]) {
+    for (int ps = 0; ps < NP; ps++) {
+        const uint32_t t = tw + FA_TQ * ps + l16;
+        if (t >= count) {
             continue;
         }
         if (splits == 1) {
             const float inv = 1.0f / l[ps];
             if (xs) {
-                const float* gm = gmax[t0[ps] - tw + l16];
+                const float* gm = gmax[FA_TQ * ps + l16];
                 const int e = row_exponent(fmaxf(fmaxf(gm[0], gm[1]), fmaxf(gm[2], gm[3])));
-                if (g == 0 && (wave & 3) == 0) {
+                if (g == 0 && wave == 0) {
                     xs_scale[t * LH_KV_HEADS + kvh] = exp2i(-e);
                 }
                 const float f = exp2i(e);
@@ -1332,29 +1351,32 @@ extern "C" int lh_launch_attention_mfma(const float* q, const float* kcache_laye
         (xs && (xs_tokens < count || !xs_scale))) {
         return -1;
     }
-    // KV splits so that about 256 workgroups run (one per CU), at most one
-    // per block of the longest tile (a 256-token chunk with no prefix runs 4
-    // splits of one block: measured 2.7 us per layer faster than 2 splits of
-    // two blocks, the merge included).
-    const bool wide = length >= lh::WIDE_MIN_LENGTH && count >= lh::WIDE_MIN_COUNT;
-    const uint32_t per_wg = wide ? lh::WIDE_WG : 2 * lh::FA_TQ;
-    const uint32_t tiles = (count + per_wg - 1) / per_wg;
+    // KV splits so that about 256 workgroups run, at most one per block of the
+    // longest tile (a 256-token chunk with no prefix runs 4 splits of one
+    // block: measured 2.7 us per layer faster than 2 splits of two blocks, the
+    // merge included) and the merge's 32. The long variant takes up to twice
+    // as many, two per CU, while a split keeps four blocks.
+    const bool far = length >= lh::FA_LONG_LENGTH;
+    const uint32_t tiles = (count + lh::FA_WG - 1) / lh::FA_WG;
     const uint32_t nb = (length + count + LH_ATTN_BLOCK - 1) / LH_ATTN_BLOCK;
     uint32_t splits = 256 / (tiles * LH_KV_HEADS);
-    const uint32_t by_length = nb;
-    splits = splits < by_length ? splits : by_length;
+    if (far) {
+        const uint32_t two = 512 / (tiles * LH_KV_HEADS), four = nb / 4;
+        const uint32_t most = two < four ? two : four;
+        splits = splits > most ? splits : most;
+        splits = splits < 32 ? splits : 32;
+    }
+    splits = splits < nb ? splits : nb;
     splits = splits ? splits : 1;
-    if (wide) {
-        hipLaunchKernelGGL(lh::k_attn_mfma_wide, dim3(tiles * LH_KV_HEADS * splits), dim3(512), 0,
-            s, q, kcache_layer, vcache_layer, length, count, capacity, PM, PT, PA, out, xs,
-            xs_tokens, xs_scale);
+    const dim3 wgs(tiles * LH_KV_HEADS * splits);
+    if (far) {
+        hipLaunchKernelGGL(lh::k_attn_mfma_long, wgs, dim3(256), 0, s, q, kcache_layer,
+            vcache_layer, length, count, capacity, PM, PT, PA, out, xs, xs_tokens, xs_scale);
     } else {
-        hipLaunchKernelGGL(lh::k_attn_mfma, dim3(tiles * LH_KV_HEADS * splits), dim3(512), 0, s,
-            q, kcache_layer, vcache_layer, length, count, capacity, PM, PT, PA, out, xs,
-            xs_tokens, xs_scale);
+        hipLaunchKernelGGL(lh::k_attn_mfma, wgs, dim3(512), 0, s, q, kcache_layer, vcache_layer,
+            length, count, capacity, PM, PT, PA, out, xs, xs_tokens, xs_scale);
     }
     if (splits > 1) {
-        static_assert(256 / LH_KV_HEADS <= 32, "at most 32 splits");
         const dim3 grid(count * LH_HEADS / 4);
         if (splits <= 4) {
             hipLaunchKernelGGL(lh::k_attn_merge<4>, grid, dim3(256), 0, s, PM, PT, PA, capacity,
