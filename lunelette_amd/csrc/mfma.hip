@@ -13,8 +13,8 @@
 //   BF16 or FP16 (v_cvt_scalef32_pk_{bf16,f16}_fp8, unit scale: every E4M3FN
 //   value has at most 4 significant bits and fits either type). The plane
 //   products accumulate in FP32.
-// - k_gemm_bf16 / k_gemm_f16: a 256-thread workgroup owns 64 tokens x 256
-//   weight rows of one K split; each wave owns 64 weight rows and all 64
+// - k_gemm_bf16: a 256-thread workgroup owns 64 tokens x 256 weight rows of one
+//   K split (k_gemm_*_n3: 192); each wave owns 64 (48) weight rows and all 64
 //   tokens (4 x 4 MFMA tiles). Per 64-column stage the activation tile (64 tokens x P planes,
 //   8P KB) goes to LDS by direct loads (global_load_lds_dwordx4) in
 //   fragment-major order, so each v_mfma_f32_16x16x32_{bf16,f16} A operand is
@@ -142,14 +142,6 @@ __host__ __device__ inline uint32_t stream_segments(uint32_t c, uint32_t stages,
         stream_group(c * stages, units, groups) + 1;
 }
 
-// Segments of column c (256 rows) of the down projection (3072 rows, 9216
-// columns) over `groups` stream-K groups.
-__device__ __forceinline__ uint32_t down_segments(uint32_t c, uint32_t groups)
-{
-    constexpr uint32_t STAGES = LH_INNER / BK, UNITS = LH_HIDDEN / GN * STAGES;
-    return stream_segments(c, STAGES, UNITS, groups);
-}
-
 // xs[p][m][k] for p < 3 from FP32 rows, no normalization. grid (count,
 // ceil(width / 2048)), block 256: thread j of the row takes columns
 // 8j .. 8j+7 (width a multiple of 8, rows 16-byte aligned).
@@ -176,17 +168,14 @@ k_split(const float* __restrict__ x, uint16_t* __restrict__ xs, uint32_t width,
 // decode kernels compute, written as the next GEMM's input planes: with F16,
 // scaled by the row's power of two 2^e and split into two FP16 planes, with
 // out_scale[t] = 2^-e to undo it on the GEMM's output; otherwise the three
-// exact BF16 planes (out_scale unused). The partials carry their own
-// groups > 0: the partials are the down projection's stream-K partials of
-// that many groups, each column summing only its segments. S = 0
+// exact BF16 planes (out_scale unused). S = 0
 // only normalizes (the first layer's input norm). grid (count), block 768:
 // thread i owns columns 4i .. 4i+3.
 template <int S, bool F16>
 __global__ void __launch_bounds__(768)
 k_residual_norm_split(const float* __restrict__ partial, size_t split_stride, float scale,
     float* __restrict__ x, const float* __restrict__ gamma,
-    uint16_t* __restrict__ xs, float* __restrict__ out_scale, uint32_t stride_tokens,
-    uint32_t groups)
+    uint16_t* __restrict__ xs, float* __restrict__ out_scale, uint32_t stride_tokens)
 {
     // Row in the [chunk][quad][lane] 16-byte-word layout: lane l's 16 values
     // of chunk c (columns c*1024 + 16l .. +15) are words (4c + q)*64 + l.
@@ -199,9 +188,7 @@ k_residual_norm_split(const float* __restrict__ partial, size_t split_stride, fl
     float4 v = xr[tid];
     if constexpr (S > 0) {
         const float4* pt = reinterpret_cast<const float4*>(partial + (size_t)t * LH_HIDDEN) + tid;
-        const float4 acc = groups
-            ? sum_segments<S>(pt, split_stride / 4, down_segments(tid / 64, groups))
-            : sum_splits<S>(pt, split_stride / 4);
+        const float4 acc = sum_splits<S>(pt, split_stride / 4);
         v.x = v.x + acc.x * scale;
         v.y = v.y + acc.y * scale;
         v.z = v.z + acc.z * scale;
@@ -452,52 +439,27 @@ __device__ __forceinline__ void store_tile(const floatx4 (&acc)[4][NF], float* _
     }
 }
 
-// store_tile, or with add the tile added to what the same lanes stored there
-// before (each element is read back only by the lane that wrote it).
-template <int NF>
-__device__ __forceinline__ void fold_tile(const floatx4 (&acc)[4][NF], float* __restrict__ o,
-    uint32_t N, uint32_t m0, uint32_t n0, uint32_t count, uint32_t lane, bool add)
-{
-    if (!add) {
-        store_tile<NF>(acc, o, N, m0, n0, count, lane);
-        return;
-    }
-    const uint32_t g = lane >> 4, l16 = lane & 15;
-#pragma unroll
-    for (int mf = 0; mf < 4; mf++) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const uint32_t m = m0 + 16 * mf + 4 * g + r;
-            if (m < count) {
-#pragma unroll
-                for (int nf = 0; nf < NF; nf++) {
-                    float* const e = o + (size_t)m * N + n0 + 16 * nf + l16;
-                    *e = *e + acc[mf][nf][r];
-                }
-            }
-        }
-    }
-}
-
 // P activation planes (PLANES_BF16 or PLANES_F16) of the same layout
 // xs[p][m][k]. Each wave owns 16 NF weight rows, the workgroup 64 NF (256 or
 // 192). grid: n_tiles * m_tiles * splits workgroups of 256 threads, two
 // resident per CU; (n_tiles * splits) a multiple of 8. W0 holds rows
 // [0, boundary), W1 rows [boundary, N) (gate|up as two tensors); boundary a
 // multiple of 64 NF.
-// out: P[s][m][n] with split stride stride_tokens * N; token rows >= count
+// out: P[s][m][n] with split stride m_tiles * 64 * N; token rows >= count
 // are not written (their activation rows, < m_tiles * 64 <= stride_tokens,
 // are read).
 //
-// With gscale, the planes of token m's K split s carry the power of two
-// 1/gscale[m][s] (row stride `splits`; the attention's output for the o
-// projection): the split's products are multiplied by gscale[m][s] (exact)
-// before the store, so the partials leave unscaled.
-template <int P, int NF>
+// With gscale, the planes of token m's K granule j (GS stages of columns each;
+// `grans` granules, the row stride) carry the power of two 1/gscale[m][j]: the
+// products of a granule are multiplied by gscale[m][j] (exact) before they join
+// the sum, so the partials leave unscaled. A split lies within one granule or
+// (FOLD) takes whole granules, whose scaled sums add up in a second register
+// tile.
+template <int P, int NF, bool FOLD = false>
 __device__ __forceinline__ void gemm_tile(const uint8_t* __restrict__ W0,
     const uint8_t* __restrict__ W1, uint32_t boundary, uint32_t N, uint32_t K,
     const uint16_t* __restrict__ xs, uint32_t stride_tokens, uint32_t count, uint32_t m_tiles,
-    uint32_t splits, const float* __restrict__ gscale, float* __restrict__ out)
+    uint32_t splits, const float* __restrict__ gscale, uint32_t grans, float* __restrict__ out)
 {
     constexpr uint32_t WN = 16 * NF, TN = 4 * WN;   // weight rows per wave, per workgroup
     static_assert(P == PLANES_BF16 || P == PLANES_F16, "plane format");
@@ -544,6 +506,30 @@ __device__ __forceinline__ void gemm_tile(const uint8_t* __restrict__ W0,
     };
     floatx4 acc[4][NF];
     zero_tile<NF>(acc);
+    floatx4 sum[FOLD ? 4 : 1][FOLD ? NF : 1];
+    // acc (or the sum) += the granule's products times their factors. Rows past
+    // count read a stale factor and are not stored.
+    const uint32_t gstages = gscale ? K / BK / grans : 0;
+    auto scale_granule = [&](uint32_t st) {
+        const uint32_t j = (s * steps + st) / gstages;
+#pragma unroll
+        for (int mf = 0; mf < 4; mf++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float f = gscale[(size_t)(m0 + 16 * mf + 4 * g + r) * grans + j];
+#pragma unroll
+                for (int nf = 0; nf < NF; nf++) {
+                    if constexpr (FOLD) {
+                        sum[mf][nf][r] = (st < gstages ? 0.0f : sum[mf][nf][r]) +
+                            acc[mf][nf][r] * f;
+                        acc[mf][nf][r] = 0.0f;
+                    } else {
+                        acc[mf][nf][r] *= f;
+                    }
+                }
+            }
+        }
+    };
     // Double-buffered stages: the next stage's activation (direct to LDS) and
     // weight loads are issued after the barrier that ends every read of the
     // LDS buffer they overwrite, and complete (s_waitcnt 0 + barrier) before
@@ -563,6 +549,9 @@ __device__ __forceinline__ void gemm_tile(const uint8_t* __restrict__ W0,
             load_w((st + 1) * BK);
         }
         gemm_stage<P, NF>(As0, wc, lane, acc);
+        if (FOLD && (st + 1) % gstages == 0) {
+            scale_granule(st);
+        }
         if (st + 1 >= steps) {
             break;
         }
@@ -577,22 +566,19 @@ __device__ __forceinline__ void gemm_tile(const uint8_t* __restrict__ W0,
             load_w((st + 2) * BK);
         }
         gemm_stage<P, NF>(As1, wc, lane, acc);
-    }
-    if (gscale) {
-        // Rows past count read a stale factor and are not stored.
-#pragma unroll
-        for (int mf = 0; mf < 4; mf++) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float f = gscale[(size_t)(m0 + 16 * mf + 4 * g + r) * splits + s];
-#pragma unroll
-                for (int nf = 0; nf < NF; nf++) {
-                    acc[mf][nf][r] *= f;
-                }
-            }
+        if (FOLD && (st + 2) % gstages == 0) {
+            scale_granule(st + 1);
         }
     }
-    store_tile<NF>(acc, out + (size_t)s * stride_tokens * N, N, m0, n0, count, lane);
+    float* const dst = out + (size_t)s * m_tiles * GM * N;
+    if constexpr (FOLD) {
+        store_tile<NF>(sum, dst, N, m0, n0, count, lane);
+    } else {
+        if (gscale) {
+            scale_granule(0);
+        }
+        store_tile<NF>(acc, dst, N, m0, n0, count, lane);
+    }
 }
 
 // gemm_tile over a stream-K partition: grid 8 * gpx * m_tiles workgroups of
@@ -601,45 +587,24 @@ __device__ __forceinline__ void gemm_tile(const uint8_t* __restrict__ W0,
 // L2. A workgroup runs its group's units back to back, the next unit's loads
 // in flight during the current one across column boundaries, and writes one
 // partial per column it covers, into slot (group - first group of the
-// column): P[slot][m][n], slot stride stride_tokens * N. A column's
+// column): P[slot][m][n], slot stride m_tiles * 64 * N. A column's
 // segments are its slots 0 .. stream_segments - 1, in K order; higher slots
 // are not written for it. Every workgroup holds the same work to within one
 // unit, so the launch has no partial last round.
-//
-// With gscale, the planes of token m's K granule j (K / GRANULES columns)
-// carry the power of two 1/gscale[m][j] (k_split_silu): the accumulator is
-// kept in units of the current granule's planes, multiplied by
-// gscale[m][j] / gscale[m][j+1] where a segment crosses into the next
-// granule and by gscale[m][j] before it is stored, so the partials are
-// unscaled. The factors are powers of two (exact products); the workgroup's
-// 64 x GRANULES factors are staged in LDS before the first stage.
-// The accumulator holds at most about 2^38 in its granule's units (576
-// products of a plane value below 2^15 and a weight below 2^9), so a ratio
-// above 2^64 could overflow it (a granule whose largest value is more than
-// 2^64 below its predecessor's, e.g. SiLU of very negative gates). Where a
-// lane's rows meet such a ratio, its wave folds the unscaled accumulator into
-// the column's partial in memory instead and restarts from zero; the column's
-// last store then adds to what was folded (each lane re-reads only what it
-// wrote itself).
-constexpr float WIDE_RATIO = 0x1p64f;
-constexpr uint32_t GRANULES = 16;
-static_assert(GRANULES == DOWN_SPLITS, "the down input's scale granules");
-
 template <int P>
 __device__ __forceinline__ void gemm_stream_tile(const uint8_t* __restrict__ W0,
     const uint8_t* __restrict__ W1, uint32_t boundary, uint32_t N, uint32_t K,
     const uint16_t* __restrict__ xs, uint32_t stride_tokens, uint32_t count, uint32_t m_tiles,
-    uint32_t gpx, const float* __restrict__ gscale, float* __restrict__ out)
+    uint32_t gpx, float* __restrict__ out)
 {
     static_assert(P == PLANES_BF16 || P == PLANES_F16, "plane format");
     constexpr uint32_t A_FRAGS = 4 * P * 2;
     constexpr uint32_t PW = A_FRAGS / 4;
     __shared__ __attribute__((aligned(1024))) uint8_t As0[A_FRAGS * 1024];
     __shared__ __attribute__((aligned(1024))) uint8_t As1[A_FRAGS * 1024];
-    __shared__ float4 gs[GM * GRANULES / 4];
     const uint32_t xcd = blockIdx.x & 7u, q = blockIdx.x >> 3;
     const uint32_t mt = q % m_tiles, groups = 8 * gpx, G = xcd * gpx + q / m_tiles;
-    const uint32_t stages = K / BK, units = N / GN * stages, gstages = stages / GRANULES;
+    const uint32_t stages = K / BK, units = N / GN * stages;
     const uint32_t u0 = stream_begin(G, units, groups), u1 = stream_begin(G + 1, units, groups);
     if (u0 >= u1) {
         return;
@@ -647,11 +612,6 @@ __device__ __forceinline__ void gemm_stream_tile(const uint8_t* __restrict__ W0,
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t g = lane >> 4, l16 = lane & 15;
     const uint32_t m0 = mt * GM;
-    if (gscale) {
-        // Rows past count take 1 (their products are never stored).
-        const float4 v = reinterpret_cast<const float4*>(gscale + (size_t)m0 * GRANULES)[tid];
-        gs[tid] = m0 + tid / 4 < count ? v : make_float4(1.f, 1.f, 1.f, 1.f);
-    }
     const size_t plane = (size_t)stride_tokens * K;
     const uint16_t* abase[PW];
 #pragma unroll
@@ -679,50 +639,13 @@ __device__ __forceinline__ void gemm_stream_tile(const uint8_t* __restrict__ W0,
     };
     floatx4 acc[4][4];
     zero_tile<4>(acc);
-    // Whether this wave has folded part of the current column into memory.
-    bool folded = false;
     // A column's partial leaves after its last stage or the range's last unit.
     auto finish = [&](uint32_t u) {
-        const uint32_t nt = u / stages, st = u - nt * stages;
-        const bool last = u + 1 == u1 || st + 1 == stages;
-        float* const dst = out + (size_t)(G - stream_group(nt * stages, units, groups)) *
-            stride_tokens * N;
-        if (gscale && (last || (st + 1) % gstages == 0)) {
-            const uint32_t j = st / gstages;
-            const float* gf = reinterpret_cast<const float*>(gs);
-            bool wide = false;
-            if (!last) {
-#pragma unroll
-                for (int mf = 0; mf < 4; mf++) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const float* row = gf + (16 * mf + 4 * g + r) * GRANULES;
-                        wide = wide || row[j] > WIDE_RATIO * row[j + 1];
-                    }
-                }
-                wide = __builtin_amdgcn_ballot_w64(wide) != 0;
-            }
-#pragma unroll
-            for (int mf = 0; mf < 4; mf++) {
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float* row = gf + (16 * mf + 4 * g + r) * GRANULES;
-                    const float f = last || wide ? row[j] : row[j] / row[j + 1];
-#pragma unroll
-                    for (int nf = 0; nf < 4; nf++) {
-                        acc[mf][nf][r] *= f;
-                    }
-                }
-            }
-            if (wide) {
-                fold_tile<4>(acc, dst, N, m0, nt * GN + wave * 64, count, lane, folded);
-                folded = true;
-                zero_tile<4>(acc);
-            }
-        }
-        if (last) {
-            fold_tile<4>(acc, dst, N, m0, nt * GN + wave * 64, count, lane, folded);
-            folded = false;
+        const uint32_t nt = u / stages;
+        if (u + 1 == u1 || u + 1 - nt * stages == stages) {
+            float* const dst = out + (size_t)(G - stream_group(nt * stages, units, groups)) *
+                m_tiles * GM * N;
+            store_tile<4>(acc, dst, N, m0, nt * GN + wave * 64, count, lane);
             zero_tile<4>(acc);
         }
     };
@@ -769,7 +692,7 @@ k_gemm_bf16(const uint8_t* __restrict__ W0, const uint8_t* __restrict__ W1, uint
     uint32_t count, uint32_t m_tiles, uint32_t splits, float* __restrict__ out)
 {
     gemm_tile<PLANES_BF16, 4>(W0, W1, boundary, N, K, xs, stride_tokens, count, m_tiles, splits,
-        nullptr, out);
+        nullptr, 0, out);
 }
 
 // 192-row workgroup tiles (48 rows per wave): q|k|v at 4 K splits and o at
@@ -781,58 +704,55 @@ k_gemm_bf16_n3(const uint8_t* __restrict__ W0, const uint8_t* __restrict__ W1, u
     uint32_t count, uint32_t m_tiles, uint32_t splits, float* __restrict__ out)
 {
     gemm_tile<PLANES_BF16, 3>(W0, W1, boundary, N, K, xs, stride_tokens, count, m_tiles, splits,
-        nullptr, out);
-}
-
-__global__ void __launch_bounds__(256, 2)
-k_gemm_f16(const uint8_t* __restrict__ W0, const uint8_t* __restrict__ W1, uint32_t boundary,
-    uint32_t N, uint32_t K, const uint16_t* __restrict__ xs, uint32_t stride_tokens,
-    uint32_t count, uint32_t m_tiles, uint32_t splits, const float* __restrict__ gscale,
-    float* __restrict__ out)
-{
-    gemm_tile<PLANES_F16, 4>(W0, W1, boundary, N, K, xs, stride_tokens, count, m_tiles, splits,
-        gscale, out);
+        nullptr, 0, out);
 }
 
 __global__ void __launch_bounds__(256, 2)
 k_gemm_f16_n3(const uint8_t* __restrict__ W0, const uint8_t* __restrict__ W1, uint32_t boundary,
     uint32_t N, uint32_t K, const uint16_t* __restrict__ xs, uint32_t stride_tokens,
     uint32_t count, uint32_t m_tiles, uint32_t splits, const float* __restrict__ gscale,
-    float* __restrict__ out)
+    uint32_t grans, float* __restrict__ out)
 {
     gemm_tile<PLANES_F16, 3>(W0, W1, boundary, N, K, xs, stride_tokens, count, m_tiles, splits,
-        gscale, out);
+        gscale, grans, out);
+}
+
+__global__ void __launch_bounds__(256, 2)
+k_gemm_f16_n3_fold(const uint8_t* __restrict__ W0, const uint8_t* __restrict__ W1,
+    uint32_t boundary, uint32_t N, uint32_t K, const uint16_t* __restrict__ xs,
+    uint32_t stride_tokens, uint32_t count, uint32_t m_tiles, uint32_t splits,
+    const float* __restrict__ gscale, uint32_t grans, float* __restrict__ out)
+{
+    gemm_tile<PLANES_F16, 3, true>(W0, W1, boundary, N, K, xs, stride_tokens, count, m_tiles,
+        splits, gscale, grans, out);
 }
 
 __global__ void __launch_bounds__(256, 2)
 k_gemm_f16_stream(const uint8_t* __restrict__ W0, const uint8_t* __restrict__ W1,
     uint32_t boundary, uint32_t N, uint32_t K, const uint16_t* __restrict__ xs,
     uint32_t stride_tokens, uint32_t count, uint32_t m_tiles, uint32_t gpx,
-    const float* __restrict__ gscale, float* __restrict__ out)
+    float* __restrict__ out)
 {
     gemm_stream_tile<PLANES_F16>(W0, W1, boundary, N, K, xs, stride_tokens, count, m_tiles, gpx,
-        gscale, out);
+        out);
 }
 
 // x[i] = x[i] + scale * (((p0 + p1) + p2) + ...) (deterministic split-K
 // combine with the residual add, src/metal_encode.m:160,175); without the
 // residual, x[i] = scale * (...). Partials P[s][i] with split stride
-// split_stride, or (groups > 0) the down projection's stream-K partials,
-// each column's segments only; i runs over count * rows in float4 units
-// (rows4 = rows / 4 per token). grid ceil(count * rows / 1024), block 256.
+// split_stride; i runs over count * rows in float4 units. grid
+// ceil(count * rows / 1024), block 256.
 template <int S>
 __global__ void __launch_bounds__(256)
 k_combine_residual(const float* __restrict__ partial, size_t split_stride, size_t n4, float scale,
-    uint32_t rows4, float* __restrict__ x, int residual, uint32_t groups)
+    float* __restrict__ x, int residual)
 {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n4) {
         return;
     }
     const float4* pi = reinterpret_cast<const float4*>(partial) + i;
-    const float4 acc = groups
-        ? sum_segments<S>(pi, split_stride / 4, down_segments((uint32_t)(i % rows4) / 64, groups))
-        : sum_splits<S>(pi, split_stride / 4);
+    const float4 acc = sum_splits<S>(pi, split_stride / 4);
     float4* xr = reinterpret_cast<float4*>(x) + i;
     float4 v = make_float4(acc.x * scale, acc.y * scale, acc.z * scale, acc.w * scale);
     if (residual) {
@@ -863,10 +783,17 @@ static uint32_t padded_block(const lh_workspace* ws)
     return (uint32_t)((ws->block + SPLIT_ROWS - 1) / SPLIT_ROWS * SPLIT_ROWS);
 }
 
-// Partial buffer: four 18432-wide splits per token (or more, narrower ones).
+// Partial buffer: four 18432-wide splits per token (or more, narrower ones, or
+// of fewer tokens).
 static size_t partial_floats(uint32_t B)
 {
     return (size_t)4 * B * MAX_N;
+}
+
+// Token rows of a partial: the call's whole 64-token tiles.
+static uint32_t partial_rows(uint32_t count)
+{
+    return (count + GM - 1) / GM * GM;
 }
 
 // Bytes of the activation planes: three BF16 (or two FP16) planes of up to
@@ -961,41 +888,44 @@ static int split_rows(const float* x, uint16_t* xs, uint32_t width, uint32_t cou
     return launched_ok("split");
 }
 
-// x = x + scale * sum of `splits` partials (groups > 0: the down projection's
-// stream-K partials; 0 splits: x unchanged), then
+// x = x + scale * sum of `splits` partials (0 splits: x unchanged), then
 // the RMSNorm of x with gamma as the next GEMM's input planes in xs: two FP16
 // planes with their row scales in out_scale, or (out_scale NULL) three BF16
 // planes; rows of 3072.
 static int residual_norm_split(const float* partial, uint32_t splits, uint32_t stride,
     float scale, float* x, const float* gamma, uint16_t* xs, float* out_scale, uint32_t count,
-    hipStream_t s, uint32_t groups = 0)
+    hipStream_t s)
 {
     return with_splits<true>(splits, "residual norm split", [&](auto S) {
         if (out_scale) {
             hipLaunchKernelGGL((k_residual_norm_split<decltype(S)::value, true>), dim3(count),
-                dim3(768), 0, s, partial, (size_t)stride * LH_HIDDEN, scale, x, gamma, xs,
-                out_scale, stride, groups);
+                dim3(768), 0, s, partial, (size_t)partial_rows(count) * LH_HIDDEN, scale, x, gamma, xs,
+                out_scale, stride);
         } else {
             hipLaunchKernelGGL((k_residual_norm_split<decltype(S)::value, false>), dim3(count),
-                dim3(768), 0, s, partial, (size_t)stride * LH_HIDDEN, scale, x, gamma, xs,
-                out_scale, stride, groups);
+                dim3(768), 0, s, partial, (size_t)partial_rows(count) * LH_HIDDEN, scale, x, gamma, xs,
+                out_scale, stride);
         }
     });
 }
 
 // P[s][m][n] for n < N over `splits` equal K ranges from `planes` activation
-// planes (PLANES_BF16 or PLANES_F16). N and boundary multiples of 256, K a
-// multiple of 64*splits, (N/256 * splits) a multiple of 8.
+// planes (PLANES_BF16 or PLANES_F16), nf 16-row operand tiles per wave (FP16
+// planes: 3). gscale: the planes' power of two per (token, K granule) of `grans`
+// granules; a split lies in one granule or takes whole ones. N and boundary
+// multiples of 64 nf, K a multiple of 64*splits, (N/(64 nf) * splits) a multiple
+// of 8.
 static int gemm(int planes, const uint8_t* W0, const uint8_t* W1, uint32_t boundary, uint32_t N,
     uint32_t K, const uint16_t* xs, uint32_t stride, uint32_t count, uint32_t splits, float* out,
-    hipStream_t s, const float* gscale = nullptr, uint32_t nf = 4)
+    hipStream_t s, uint32_t nf = 4, const float* gscale = nullptr, uint32_t grans = 0)
 {
     const uint32_t tn = 64 * nf;   // weight rows per workgroup
     const uint32_t n_tiles = N / tn;
     const uint32_t m_tiles = (count + GM - 1) / GM;
-    if (!count || !splits || (nf != 3 && nf != 4) || N % tn || (n_tiles * splits) % 8 ||
-        K % (BK * splits) || boundary % tn || m_tiles * GM > stride ||
-        (size_t)splits * stride * N > partial_floats(stride)) {
+    if (!count || !splits || (nf != 3 && nf != 4) || (planes == PLANES_F16 && nf != 3) || N % tn ||
+        (n_tiles * splits) % 8 || K % (BK * splits) || boundary % tn || m_tiles * GM > stride ||
+        (size_t)splits * m_tiles * GM * N > partial_floats(stride) ||
+        (gscale && (!grans || K % (BK * grans) || (splits % grans && grans % splits)))) {
         lh_set_error("gemm: unsupported shape N=%u K=%u splits=%u", N, K, splits);
         return -1;
     }
@@ -1004,8 +934,9 @@ static int gemm(int planes, const uint8_t* W0, const uint8_t* W1, uint32_t bound
         hipLaunchKernelGGL(nf == 4 ? k_gemm_bf16 : k_gemm_bf16_n3, grid, dim3(256), 0, s,
             W0, W1 ? W1 : W0, boundary, N, K, xs, stride, count, m_tiles, splits, out);
     } else {
-        hipLaunchKernelGGL(nf == 4 ? k_gemm_f16 : k_gemm_f16_n3, grid, dim3(256), 0, s,
-            W0, W1 ? W1 : W0, boundary, N, K, xs, stride, count, m_tiles, splits, gscale, out);
+        hipLaunchKernelGGL(gscale && grans > splits ? k_gemm_f16_n3_fold : k_gemm_f16_n3, grid,
+            dim3(256), 0, s, W0, W1 ? W1 : W0, boundary, N, K, xs, stride, count, m_tiles, splits,
+            gscale, grans, out);
     }
     return launched_ok("gemm");
 }
@@ -1016,13 +947,12 @@ static int gemm(int planes, const uint8_t* W0, const uint8_t* W1, uint32_t bound
 // slot count in *slots and the group count in *groups.
 template <uint32_t MAXS>
 static int gemm_stream(const uint8_t* W0, const uint8_t* W1, uint32_t boundary, uint32_t N,
-    uint32_t K, const uint16_t* xs, uint32_t stride, uint32_t count, const float* gscale,
-    float* out, uint32_t* slots, uint32_t* groups, hipStream_t s)
+    uint32_t K, const uint16_t* xs, uint32_t stride, uint32_t count, float* out, uint32_t* slots,
+    uint32_t* groups, hipStream_t s)
 {
     const uint32_t n_tiles = N / GN;
     const uint32_t m_tiles = (count + GM - 1) / GM;
-    if (!count || N % GN || K % BK || boundary % GN || m_tiles * GM > stride || m_tiles > 64 ||
-        (gscale && K % (BK * GRANULES))) {
+    if (!count || N % GN || K % BK || boundary % GN || m_tiles * GM > stride || m_tiles > 64) {
         lh_set_error("stream gemm: unsupported shape N=%u K=%u count=%u", N, K, count);
         return -1;
     }
@@ -1033,11 +963,11 @@ static int gemm_stream(const uint8_t* W0, const uint8_t* W1, uint32_t boundary, 
         for (uint32_t c = 0; c < n_tiles; c++) {
             most = std::max(most, stream_segments(c, stages, units, ng));
         }
-        if (most > MAXS || (size_t)most * stride * N > partial_floats(stride)) {
+        if (most > MAXS || (size_t)most * m_tiles * GM * N > partial_floats(stride)) {
             continue;
         }
         hipLaunchKernelGGL(k_gemm_f16_stream, dim3(ng * m_tiles), dim3(256), 0, s, W0,
-            W1 ? W1 : W0, boundary, N, K, xs, stride, count, m_tiles, gpx, gscale, out);
+            W1 ? W1 : W0, boundary, N, K, xs, stride, count, m_tiles, gpx, out);
         *slots = most;
         *groups = ng;
         return launched_ok("stream gemm");
@@ -1047,13 +977,13 @@ static int gemm_stream(const uint8_t* W0, const uint8_t* W1, uint32_t boundary, 
 }
 
 static int combine(const float* partial, uint32_t splits, uint32_t rows, uint32_t count,
-    uint32_t stride, float scale, float* x, int residual, hipStream_t s, uint32_t groups = 0)
+    float scale, float* x, int residual, hipStream_t s)
 {
     const size_t n4 = (size_t)count * rows / 4;
     return with_splits(splits, "split-K combine", [&](auto S) {
         hipLaunchKernelGGL(k_combine_residual<decltype(S)::value>,
             dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, partial,
-            (size_t)stride * rows, n4, scale, rows / 4, x, residual, groups);
+            (size_t)partial_rows(count) * rows, n4, scale, x, residual);
     });
 }
 
@@ -1083,7 +1013,7 @@ extern "C" int lh_fp8_gemm(lh_workspace* ws, const uint8_t* d_w, float scale, co
             B, n, splits, ws->d_gemm, s)) {
         return -1;
     }
-    return combine(ws->d_gemm, splits, (uint32_t)rows, n, B, scale, d_y, 0, s);
+    return combine(ws->d_gemm, splits, (uint32_t)rows, n, scale, d_y, 0, s);
 }
 
 // A layer over at most SMALL_TOKENS tokens (mfma_small.hip): no partials; the
@@ -1149,18 +1079,19 @@ extern "C" int lh_layer_forward_mfma(const lh_layer_weights* w, float* d_x, floa
     uint16_t* xs = ws->d_split;
     float* scale_a = token_scales(ws);
     float* scale_b = group_scales(ws);
-    // K splits (measured at 256 tokens): q|k|v 4, o 8, down 16; gate|up is
-    // stream-K.
+    const uint32_t m_tiles = partial_rows(n) / GM, R = partial_rows(n);
     // q|k|v: 6144 rows, 3072 columns; scales, RoPE and the KV append in the
-    // epilogue.
-    const uint32_t sq = 4;
+    // epilogue. K splits: one token tile's 128 workgroups of 4 splits leave half
+    // of the CUs idle (50 tokens: 16.1 us, 13.7 with 8); from two tiles on, 8
+    // splits only add partials (100 tokens 17.9 and 17.8 us, 256 29.7 and 32.5).
+    const uint32_t sq = m_tiles == 1 ? 8 : 4;
     if ((!input_split &&
             residual_norm_split(NULL, 0, B, 1.0f, d_x, w->input_norm, xs, NULL, n, s)) ||
         gemm(PLANES_BF16, w->qkv, NULL, LH_QKV_ROWS, LH_QKV_ROWS, LH_HIDDEN, xs, B, n, sq, P, s,
-            nullptr, 3) ||
+            3) ||
         with_splits(sq, "qkv epilogue", [&](auto S) {
             hipLaunchKernelGGL(k_qkv_epilogue<decltype(S)::value>, dim3(n, 3), dim3(256), 0, s,
-                P, (size_t)B * LH_QKV_ROWS, make_float3(w->scale[0], w->scale[1], w->scale[2]),
+                P, (size_t)R * LH_QKV_ROWS, make_float3(w->scale[0], w->scale[1], w->scale[2]),
                 ws->d_params, ws->d_q, d_keys, d_values, C);
         })) {
         return -1;
@@ -1174,8 +1105,8 @@ extern "C" int lh_layer_forward_mfma(const lh_layer_weights* w, float* d_x, floa
     if (lh_launch_attention_mfma(ws->d_q, d_keys, d_values, ws->d_params, (uint32_t)ws->length,
             n, C, ws->d_PM, ws->d_PT, ws->d_PA, ws->d_attn, xs, B, scale_b, s) ||
         launched_ok("attention") ||
-        gemm(PLANES_F16, w->o, NULL, LH_HIDDEN, LH_HIDDEN, LH_QUERY, xs, B, n, so, P, s,
-            scale_b, 3) ||
+        gemm(PLANES_F16, w->o, NULL, LH_HIDDEN, LH_HIDDEN, LH_QUERY, xs, B, n, so, P, s, 3,
+            scale_b, LH_KV_HEADS) ||
         residual_norm_split(P, so, B, w->scale[3], d_x, w->post_norm, xs, scale_a, n, s)) {
         return -1;
     }
@@ -1183,27 +1114,28 @@ extern "C" int lh_layer_forward_mfma(const lh_layer_weights* w, float* d_x, floa
     // 27 stages, at most 3 partials per column); SiLU(gate)*up as the down
     // projection's input.
     uint32_t sg = 0, groups = 0;
-    if (gemm_stream<4>(w->gate, w->up, LH_INNER, MAX_N, LH_HIDDEN, xs, B, n, NULL, P, &sg,
+    if (gemm_stream<4>(w->gate, w->up, LH_INNER, MAX_N, LH_HIDDEN, xs, B, n, P, &sg,
             &groups, s) ||
         with_splits<false, 4>(sg, "silu split", [&](auto S) {
             hipLaunchKernelGGL(k_split_silu<decltype(S)::value>, dim3(n, DOWN_SPLITS), dim3(192),
-                0, s, P, (size_t)B * MAX_N, make_float2(w->scale[4], w->scale[5]), scale_a, xs,
+                0, s, P, (size_t)R * MAX_N, make_float2(w->scale[4], w->scale[5]), scale_a, xs,
                 scale_b, B, groups);
         })) {
         return -1;
     }
-    // down: 3072 rows, 9216 columns, stream-K (at 256 tokens 128 groups of
-    // 13-14 stages, 11-12 partials per column) with the input's granule
-    // scales applied in the GEMM; residual (and the next layer's input
-    // planes).
-    uint32_t sd = 0, dgroups = 0;
-    if (gemm_stream<16>(w->down, NULL, LH_HIDDEN, LH_HIDDEN, LH_INNER, xs, B, n, scale_b, P, &sd,
-            &dgroups, s)) {
+    // down: 3072 rows, 9216 columns in 16 K granules with a scale each; residual
+    // (and the next layer's input planes). One granule per split up to two
+    // token tiles, two from three tiles on: 256 to 512 workgroups of the same
+    // work (at 256 tokens exactly two per CU). Against a stream-K partition of
+    // 192 to 512 workgroups and 11 to 16 partials per column (50, 100, 180, 256
+    // tokens): 16.1, 22.1, 31.5, 39 -> 13.3, 19, 28.1, 31 us, and the consumer's
+    // sums 1 to 2 us less.
+    const uint32_t sd = m_tiles <= 2 ? DOWN_SPLITS : DOWN_SPLITS / 2;
+    if (gemm(PLANES_F16, w->down, NULL, LH_HIDDEN, LH_HIDDEN, LH_INNER, xs, B, n, sd, P, s, 3,
+            scale_b, DOWN_SPLITS)) {
         return -1;
     }
-    // Segment counts vary by column: sum with the 16-slot kernels.
-    sd = 16;
     return next_norm
-        ? residual_norm_split(P, sd, B, w->scale[6], d_x, next_norm, xs, NULL, n, s, dgroups)
-        : combine(P, sd, LH_HIDDEN, n, B, w->scale[6], d_x, 1, s, dgroups);
+        ? residual_norm_split(P, sd, B, w->scale[6], d_x, next_norm, xs, NULL, n, s)
+        : combine(P, sd, LH_HIDDEN, n, w->scale[6], d_x, 1, s);
 }
