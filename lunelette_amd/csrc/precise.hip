@@ -78,13 +78,13 @@ __device__ __forceinline__ uint32_t tile_row(uint32_t n)
     return EPI == EPI_RESIDUAL || n < NP ? n : n - NP + (EPI == EPI_QKV ? 64 : 0);
 }
 
-// Tiles of 16 tokens x 16 RT weight rows of a K = 1024 NCH projection.
+// Tiles of 16 TT tokens x 16 RT weight rows of a K = 1024 NCH projection.
 // Workgroup id (512 threads) takes tiles id, id + gridDim.x, ...; gridDim.x and the
 // row tiles are multiples of 8. Tile j's token tiles follow each other on XCD
 // j % 8, so a row tile's weights come from HBM once. A tile's first stage is
 // requested during the last stages of the tile before it and lands under that
 // tile's reduction and epilogue.
-template <int KIND, int NCH, int RT, int EPI>
+template <int KIND, int NCH, int TT, int RT, int EPI>
 __device__ __forceinline__ void tile_body(const TileArgs& a)
 {
     constexpr uint32_t K = NCH * LH_CHUNK, ES = KIND == K_FP8 ? 1 : 4;
@@ -102,13 +102,13 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
     __shared__ u32x4 w0[STAGE_WORDS];
     __shared__ u32x4 w1[STAGE_WORDS];
     __shared__ u32x4 w2[NB == 3 ? STAGE_WORDS : 1];
-    __shared__ __attribute__((aligned(16))) float red[8 * 16 * RS];
+    __shared__ __attribute__((aligned(16))) float red[8 * 16 * TT * RS];
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t s = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint32_t tile = blockIdx.x, tt, rt;
     // Scalar offsets of the stage loads (the tensors are below 4 GiB).
     const char* const W = EPI == EPI_GATEUP && s >= 4 ? a.W1 : a.W;
-    uint32_t src, xsrc;
+    uint32_t src, xsrc[TT];
     // Direct loads: load i of wave s fills LDS words (s * LOADS + i) * 64 + lane,
     // row n = word / ROW_WORDS; LDS word w of row n holds the row's word w ^ (n & 15).
     // Waves 0..3 load the lower half of the rows.
@@ -120,12 +120,19 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
         off[i] = tile_row<RT, EPI>(n) * K * ES + 16 * (w ^ (n & 15));
     }
     auto locate = [&](uint32_t j) {
-        const uint32_t rest = j >> 3;
-        tt = rest % a.token_tiles;
-        rt = (rest / a.token_tiles) * 8 + (j & 7);
+        const uint32_t rest = j >> 3, groups = (a.token_tiles + TT - 1) / TT;
+        tt = rest % groups * TT;
+        rt = (rest / groups) * 8 + (j & 7);
     };
     auto weights = [&]() { src = tile_base<RT, EPI>(rt) * K * ES; };
-    auto activations = [&]() { xsrc = (tt * (K >> 9) * 2048 + s * 256) * 16; };
+    // (A group's token tiles past the last repeat it; their rows lie past count.)
+    auto activations = [&]() {
+#pragma unroll
+        for (int m = 0; m < TT; m++) {
+            const uint32_t tile = tt + m < a.token_tiles ? tt + m : a.token_tiles - 1;
+            xsrc[m] = (tile * (K >> 9) * 2048 + s * 256) * 16;
+        }
+    };
     auto load_w = [&](uint32_t stage, u32x4* buf) {
         const char* p = W + __builtin_amdgcn_readfirstlane(src + stage * 512 * ES);
 #pragma unroll
@@ -133,18 +140,21 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
             __builtin_amdgcn_global_load_lds(p + off[i], buf + (s * LOADS + i) * 64, 16, 0, 0);
         }
     };
-    f32x4 xn[4], xc[4];
+    f32x4 xn[TT][4], xc[TT][4];
     auto load_x = [&](uint32_t stage) {
-        const f32x4* p = reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(a.xt) +
-            __builtin_amdgcn_readfirstlane(xsrc + stage * 2048 * 16));
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            xn[i] = p[i * 64 + lane];
+        for (int m = 0; m < TT; m++) {
+            const f32x4* p = reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(a.xt) +
+                __builtin_amdgcn_readfirstlane(xsrc[m] + stage * 2048 * 16));
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                xn[m][i] = p[i * 64 + lane];
+            }
         }
     };
     // Operand words of row tile r: row n = 16 r + lane % 16, chain 8 (lane / 16) + s.
     const uint32_t n16 = lane & 15, wbase = ((lane >> 4) * 8 + s) * WQ;
-    f32x16 acc[RT][2];
+    f32x16 acc[TT][RT][2];
     auto compute = [&](const u32x4* buf, int g) {
         u32x4 raw[RT][KIND == K_FP8 ? 1 : 4];
 #pragma unroll
@@ -181,9 +191,12 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
 #pragma unroll
-                for (int r = 0; r < RT; r++) {
-                    acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x1f32(xc[i][e], w[i & 1][r][e],
-                        acc[r][g], 0, 0, 0);
+                for (int m = 0; m < TT; m++) {
+#pragma unroll
+                    for (int r = 0; r < RT; r++) {
+                        acc[m][r][g] = __builtin_amdgcn_mfma_f32_16x16x1f32(xc[m][i][e],
+                            w[i & 1][r][e], acc[m][r][g], 0, 0, 0);
+                    }
                 }
                 __builtin_amdgcn_sched_barrier(0x6);
             }
@@ -196,7 +209,7 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
         f32x4 v[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            v[i] = p[i * 16 * RS / 4];
+            v[i] = p[i * 16 * TT * RS / 4];
         }
         return ((v[0] + v[4]) + (v[2] + v[6])) + ((v[1] + v[5]) + (v[3] + v[7]));
     };
@@ -214,8 +227,11 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
     u32x4* const bufs[3] = {w0, w1, w2};
     while (true) {
 #pragma unroll
-        for (int r = 0; r < RT; r++) {
-            acc[r][0] = acc[r][1] = f32x16{};
+        for (int m = 0; m < TT; m++) {
+#pragma unroll
+            for (int r = 0; r < RT; r++) {
+                acc[m][r][0] = acc[m][r][1] = f32x16{};
+            }
         }
         const uint32_t t0 = tt * 16, n0 = rt;
         const bool more = tile + gridDim.x < a.tiles;
@@ -232,8 +248,11 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
                 asm volatile("" ::: "memory");
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    xc[i] = xn[i];
+                for (int m = 0; m < TT; m++) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        xc[m][i] = xn[m][i];
+                    }
                 }
                 // Stage k + 1's activations, then stage k + AHEAD's weights;
                 // past this tile's last stage, the next tile's (the last
@@ -256,12 +275,15 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
         // Tree levels 32 (the two accumulators), 16 and 8 (their blocks): lane
         // holds tokens 4 (lane / 16) + k, row lane % 16 of each row tile.
 #pragma unroll
-        for (int r = 0; r < RT; r++) {
-            const f32x16 v = acc[r][0] + acc[r][1];
+        for (int m = 0; m < TT; m++) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                red[(s * 16 + 4 * (lane >> 4) + k) * RS + 16 * r + n16] =
-                    (v[k] + v[8 + k]) + (v[4 + k] + v[12 + k]);
+            for (int r = 0; r < RT; r++) {
+                const f32x16 v = acc[m][r][0] + acc[m][r][1];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    red[((s * TT + m) * 16 + 4 * (lane >> 4) + k) * RS + 16 * r + n16] =
+                        (v[k] + v[8 + k]) + (v[4 + k] + v[12 + k]);
+                }
             }
         }
         // LDS only: the next tile's first stage stays in flight.
@@ -271,7 +293,7 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
         asm volatile("" ::: "memory");
         if constexpr (EPI == EPI_RESIDUAL) {
             const uint32_t tl = tid / (4 * RT), n = tid % (4 * RT) * 4, t = t0 + tl;
-            if (tid < 64 * RT && t < a.count) {
+            if (tid < 64 * RT * TT && t < a.count) {
                 f32x4* px = reinterpret_cast<f32x4*>(a.x + (size_t)t * LH_HIDDEN +
                     n0 * 16 * RT + n);
                 const f32x4 old = *px, v = total4(tl, n);
@@ -279,7 +301,7 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
             }
         } else if constexpr (EPI == EPI_QKV) {
             const uint32_t tl = tid / (2 * RT), n = tid % (2 * RT) * 4, t = t0 + tl;
-            if (tid < 32 * RT && t < a.count) {
+            if (tid < 32 * RT * TT && t < a.count) {
                 const uint32_t pair = n0 * NP + n, head = pair >> 6, i = pair & 63;
                 const float scale = head < 32 ? a.s0 : (head < 40 ? a.s1 : a.s2);
                 const f32x4 lo = total4(tl, n) * scale, hi = total4(tl, n + NP) * scale;
@@ -314,8 +336,8 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
         } else {
             // One word of the next projection's tile order per thread. Rows
             // past count are written too (their products are never stored).
-            const uint32_t tl = tid & 15, n = (tid >> 4) * 4;
-            if (tid < 32 * RT) {
+            const uint32_t tl = tid % (16 * TT), n = tid / (16 * TT) * 4;
+            if (tid < 32 * RT * TT && t0 + tl < a.token_tiles * 16) {
                 const f32x4 g = total4(tl, n) * a.s0, u = total4(tl, n + NP) * a.s1;
                 f32x4 y;
 #pragma unroll
@@ -334,12 +356,12 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
 }
 
 // (The body is device code only: the host pass has no matrix instructions.)
-template <int KIND, int NCH, int RT, int EPI>
-__global__ void __launch_bounds__(512, 4)
+template <int KIND, int NCH, int TT, int RT, int EPI>
+__global__ void __launch_bounds__(512, TT == 1 ? 4 : 2)
 k_tile(TileArgs a)
 {
 #ifdef __HIP_DEVICE_COMPILE__
-    tile_body<KIND, NCH, RT, EPI>(a);
+    tile_body<KIND, NCH, TT, RT, EPI>(a);
 #endif
 }
 
@@ -406,8 +428,8 @@ k_norm_tile(const float* __restrict__ x, const float* __restrict__ gamma, f32x4*
 // Bound: FP32 matrix instructions, 8192 cycles per wave and block: 256 tokens
 // after 4096 positions are 17.6 GFLOP, 0.13 ms at 2 GHz, and write 285 MB of
 // partials. Measured there 0.24 ms (0.76 ms with one token per workgroup,
-// k_attn_blocks) plus 0.06 ms for the combine, which reads the partials back
-// at 4.9 TB/s; 37 tokens after 777: 19 us plus 9 (30 and 5).
+// k_attn_blocks) plus 0.04 ms for the combine, which reads the partials back;
+// 37 tokens after 777: 19 us plus 5 (30 and 5).
 //
 // grid 8 * query groups * ranges, block 256: id = (range * groups + group) * 8 +
 // kv head; a group is 16 tokens, a range `per` consecutive blocks.
@@ -697,32 +719,44 @@ static int launched()
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// Two workgroups fit a CU (128 registers, at most 76 KB of LDS).
-template <int KIND, int NCH, int RT, int EPI>
+// One token tile per workgroup: two workgroups fit a CU (128 registers, at most
+// 76 KB of LDS); more: one.
+template <int KIND, int NCH, int TT, int RT, int EPI>
 static void launch_tile(uint32_t rows, TileArgs a, hipStream_t s)
 {
-    a.tiles = rows / (16 * RT) * a.token_tiles;
-    hipLaunchKernelGGL((k_tile<KIND, NCH, RT, EPI>), dim3(a.tiles < 512 ? a.tiles : 512),
-        dim3(512), 0, s, a);
+    a.tiles = rows / (16 * RT) * ((a.token_tiles + TT - 1) / TT);
+    const uint32_t resident = TT == 1 ? 512 : 256;
+    hipLaunchKernelGGL((k_tile<KIND, NCH, TT, RT, EPI>),
+        dim3(a.tiles < resident ? a.tiles : resident), dim3(512), 0, s, a);
 }
 
 // FP8 projections take two row tiles per workgroup where that leaves no CU
 // with more of them than single ones would (the CU with the most work holds
 // ceil(workgroups / 256) workgroups): at 256 tokens 0.61 ms a layer against
 // 0.66 ms with one, at 16 tokens 77 against 62 us. Four per workgroup (one
-// resident per CU) measured the same as two at 256 tokens and worse below.
-// FP32 rows take one: their stages are four times as large.
+// resident per CU) measured the same as two at 256 tokens and worse below; two
+// or three token tiles instead were slower (37 tokens: 183 against 172 us).
+// FP32 rows, four times as large, take one row tile and up to three token
+// tiles, which then share one read of the rows (layers after 517 positions of 24,
+// 48, 64 and 90 tokens: 198, 254, 308, 408 us with one token tile, 186, 228, 290,
+// 368 us so).
 template <int KIND, int NCH, int EPI>
 static int run_tile(uint32_t rows, const TileArgs& a, hipStream_t s)
 {
-    const uint32_t single = rows / 16 * a.token_tiles;
     if constexpr (KIND == K_FP8) {
+        const uint32_t single = rows / 16 * a.token_tiles;
         if ((single / 2 + 255) / 256 * 2 <= (single + 255) / 256) {
-            launch_tile<KIND, NCH, 2, EPI>(rows, a, s);
-            return launched();
+            launch_tile<KIND, NCH, 1, 2, EPI>(rows, a, s);
+        } else {
+            launch_tile<KIND, NCH, 1, 1, EPI>(rows, a, s);
         }
+    } else if (a.token_tiles == 1) {
+        launch_tile<KIND, NCH, 1, 1, EPI>(rows, a, s);
+    } else if (a.token_tiles % 3) {
+        launch_tile<KIND, NCH, 2, 1, EPI>(rows, a, s);
+    } else {
+        launch_tile<KIND, NCH, 3, 1, EPI>(rows, a, s);
     }
-    launch_tile<KIND, NCH, 1, EPI>(rows, a, s);
     return launched();
 }
 

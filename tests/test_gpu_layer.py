@@ -115,10 +115,11 @@ def test_prefill_chunk_small(gpu, layer_host):
 
 
 @pytest.mark.parametrize("length,count", [(62, 2), (3, 4), (777, 15), (0, 16), (1000, 17),
-                                          (64, 33), (130, 130)])
+                                          (64, 33), (40, 70), (130, 130)])
 def test_multi_token_layer_tiles(gpu, layer_host, length, count):
     """The tiled projections of the precise path at the edges of their
-    16-token tiles and of the two workgroup widths, every strategy, bitwise."""
+    16-token tiles and of their workgroup shapes (one to nine token tiles, in
+    groups of one, two or three), every strategy, bitwise."""
     paths = [lh.PATH_FUSED, lh.PATH_RESIDENT]
     check_layer(gpu, layer_host, length, count, 4352,
                 paths + [lh.PATH_LOOKUP] if count < 20 else paths)
