@@ -79,9 +79,7 @@ struct CombineShared {
 // group s of each 256-block round; every quarter recomputes M and the block
 // factors, so the four workgroups of a head are independent. Bitwise the
 // schedule above (the dims never mix; groups start at multiples of 8 from
-// block 0 and add left to right across rounds). XT: out in the o projection's
-// activation tile order (lh_xt_word), n known to the host.
-template <bool XT = false>
+// block 0 and add left to right across rounds).
 __device__ __forceinline__ void attn_combine(const float* __restrict__ PM,
     const float* __restrict__ PT, const float* __restrict__ PA, uint32_t n, uint32_t capacity,
     uint32_t h, uint32_t qd, uint32_t t, float* __restrict__ out, CombineShared& sh)
@@ -94,24 +92,21 @@ __device__ __forceinline__ void attn_combine(const float* __restrict__ PM,
     const float4* pa = reinterpret_cast<const float4*>(PA + th * nbc * LH_HEAD_DIM) + 8 * qd + c;
     // A round's partial loads are clamped to the capacity, not to the valid
     // block count, so the first round's issue before the step record is
-    // read; rows past the valid count never enter arithmetic. Where n comes
-    // with the launch they are clamped to the valid blocks (48 tokens after 517
-    // positions of a 4352-position cache: 14.2 -> 5.3 us).
-    const uint32_t nb = (n + LH_ATTN_BLOCK - 1) / LH_ATTN_BLOCK;
-    const uint32_t end = XT ? nb : nbc;
+    // read; rows past the valid count never enter arithmetic.
     float4 a[GROUP];
     float m_own, t_own;
     auto load_round = [&](uint32_t r0) {
 #pragma unroll
         for (uint32_t k = 0; k < GROUP; k++) {
             const uint32_t bb = r0 + s * GROUP + k;
-            a[k] = pa[(size_t)(bb < end ? bb : end - 1) * (LH_HEAD_DIM / 4)];
+            a[k] = pa[(size_t)(bb < nbc ? bb : nbc - 1) * (LH_HEAD_DIM / 4)];
         }
-        const uint32_t bb = r0 + tid < end ? r0 + tid : end - 1;
+        const uint32_t bb = r0 + tid < nbc ? r0 + tid : nbc - 1;
         m_own = pm[bb];
         t_own = pt[bb];
     };
     load_round(0);
+    const uint32_t nb = (n + LH_ATTN_BLOCK - 1) / LH_ATTN_BLOCK;
     float M = tid < nb ? m_own : -__builtin_inff();
     for (uint32_t j = tid + ROUND; j < nb; j += ROUND) {
         M = fmaxf(M, pm[j]);
@@ -170,9 +165,8 @@ __device__ __forceinline__ void attn_combine(const float* __restrict__ PM,
         __syncthreads();
     }
     if (tid < 8) {
-        const uint32_t col = h * LH_HEAD_DIM + 32 * qd + 4 * c;
-        reinterpret_cast<float4*>(out)[XT ? lh_xt_word(t, col, LH_QUERY)
-            : ((size_t)t * LH_QUERY + col) / 4] = make_float4(A.x / T, A.y / T, A.z / T, A.w / T);
+        reinterpret_cast<float4*>(out + (size_t)t * LH_QUERY + h * LH_HEAD_DIM)[8 * qd + c] =
+            make_float4(A.x / T, A.y / T, A.z / T, A.w / T);
     }
 }
 
