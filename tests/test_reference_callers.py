@@ -21,7 +21,7 @@ REF = "/root/reference"
 
 
 def build(sources, out):
-    if not os.path.isdir(REF):
+    if not os.path.isfile(os.path.join(REF, "src", "main.c")):
         pytest.skip("the reference checkout is not present")
     if not shutil.which("gcc"):
         pytest.skip("gcc not available")
