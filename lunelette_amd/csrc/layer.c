@@ -350,6 +350,24 @@ static int layer_tiles(const lh_layer_weights *w, float *x, float *keys, float *
 #define TILES_MIN 5
 #define TILES_MIN_RESIDENT 2
 
+/* The tiled path loads 16 bytes per lane straight to LDS, which needs 16-byte
+ * addresses; tensors elsewhere stay on the row dots. */
+static int tiles_aligned(const lh_layer_weights *w, const float *x, const float *keys,
+    const float *values, int resident)
+{
+    const void *p[] = {resident ? (const void *)w->f32_qkv : (const void *)w->qkv,
+        resident ? (const void *)w->f32_o : (const void *)w->o,
+        resident ? (const void *)w->f32_gate : (const void *)w->gate,
+        resident ? (const void *)w->f32_up : (const void *)w->up,
+        resident ? (const void *)w->f32_down : (const void *)w->down,
+        w->input_norm, w->post_norm, x, keys, values};
+    uintptr_t bits = 0;
+    for (size_t i = 0; i < sizeof p / sizeof p[0]; i++) {
+        bits |= (uintptr_t)p[i];
+    }
+    return bits % 16 == 0;
+}
+
 int lh_layer_operator(int op, const lh_layer_weights *w, float *d_x, float *d_keys,
     float *d_values, lh_workspace *ws, void *stream)
 {
@@ -390,7 +408,8 @@ int lh_layer_forward(const lh_layer_weights *w, float *d_x, float *d_keys, float
         return -1;
     }
     hipStream_t s = (hipStream_t)stream;
-    const int tiles = ws->count >= (path == LH_PATH_RESIDENT ? TILES_MIN_RESIDENT : TILES_MIN);
+    const int tiles = ws->count >= (path == LH_PATH_RESIDENT ? TILES_MIN_RESIDENT : TILES_MIN) &&
+        tiles_aligned(w, d_x, d_keys, d_values, path == LH_PATH_RESIDENT);
     switch (path) {
     case LH_PATH_FUSED:
         return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 0, s)

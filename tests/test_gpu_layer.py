@@ -125,6 +125,39 @@ def test_multi_token_layer_tiles(gpu, layer_host, length, count):
                 paths + [lh.PATH_LOOKUP] if count < 20 else paths)
 
 
+def test_multi_token_layer_unaligned_weights(gpu, layer_host):
+    """FP8 weight tensors 4 bytes past a 16-byte boundary take the row dots:
+    the same bits."""
+    length, count, capacity = 70, 9, 256
+    x = syn.normal_f32(SEED, 9021, count * 3072)
+    kpm = syn.normal_f32(SEED, 9022, length * 1024).reshape(length, 1024)
+    vpm = syn.normal_f32(SEED, 9023, length * 1024).reshape(length, 1024)
+    want = run_layer(gpu, layer_host, x, kpm, vpm, length, count, capacity, lh.PATH_FUSED)
+    dev = gpu_util.DeviceLayer(layer_host)
+    weights = dev.weights
+    moved = []
+    for name in ("o", "gate", "down"):
+        codes = np.ascontiguousarray(layer_host[name], np.uint8).reshape(-1)
+        buf = lh.DeviceBuffer.from_array(np.concatenate([np.zeros(4, np.uint8), codes]))
+        moved.append(buf)
+        setattr(getattr(weights, "contents", weights), name, buf.ptr + 4)
+    keys = lh.DeviceBuffer.from_array(gpu_util.keys_to_device(kpm, capacity))
+    values = lh.DeviceBuffer.from_array(gpu_util.kv_to_device_layout(vpm, capacity))
+    d_x = lh.DeviceBuffer.from_array(x)
+    ws = gpu.lh_workspace_create(capacity, count)
+    assert ws, lh.last_error()
+    try:
+        ids = np.zeros(count, np.int64)
+        lh.check(gpu.lh_workspace_set_tokens(ws, ids.ctypes.data_as(lh.c_int64_p), length, count,
+                                             None), "set_tokens")
+        lh.check(gpu.lh_layer_forward(weights, d_x.ptr, keys.ptr, values.ptr, ws, lh.PATH_FUSED,
+                                      None), "layer_forward")
+        lh.check(gpu.lh_device_synchronize())
+        assert np.array_equal(bits(d_x.download(np.float32)), bits(want[0]))
+    finally:
+        gpu.lh_workspace_destroy(ws)
+
+
 @pytest.mark.parametrize("length,count", [(0, 5), (70, 20), (120, 41)])
 def test_multi_token_layer_nonfinite_token(gpu, layer_host, length, count):
     """A token whose input is infinite leaves NaN values in the cache; the
