@@ -31,6 +31,8 @@
 
 #include <pthread.h>
 
+#include <algorithm>
+
 namespace lh {
 
 // grid (8 * nblk * count): workgroup id = (t * nblk + b) * 8 + kvh, so every
@@ -910,10 +912,13 @@ k_attn_mfma(const float* __restrict__ q, const float* __restrict__ kcache,
 // and blocks that raise no maximum the rescaling of O.
 // Measured (kernel trace), k_attn_mfma and the former 64-token variant before:
 // 64 tokens after 15872 positions 86 -> 70 us (and 3 us more in the merge of
-// twice as many splits), 256 after 4096 80 -> 77 us; the layer of 130 tokens after
-// 5000 231 -> 214 us; with one workgroup per CU 80 and 88 us. After short prefixes its 4-wave workgroups lose (201 tokens after 256:
-// 19.2 against 17.9 us).
-constexpr uint32_t FA_LONG_LENGTH = 2048;   // prefix from which it pays
+// twice as many splits), 256 after 4096 80 -> 77 us (86 us for it at the lower
+// clock of another box); the layer of 130 tokens after 5000 231 -> 214 us. With
+// one workgroup per CU these took 80 and 88 us: lh_attention_mfma_plan picks it
+// where two fit. After short prefixes its 4-wave workgroups lose (201 tokens after
+// 256: 19.2 against 17.9 us).
+constexpr uint32_t FA_LONG_LENGTH = 2048;     // prefix from which it can pay
+constexpr uint32_t FA_LONG_ONE_TILE = 4096;   // and for up to 32 tokens does
 
 // The thread id again, where a value held for it across the block loop would
 // spill.
@@ -1342,6 +1347,41 @@ k_attn_merge(const float* __restrict__ PM, const float* __restrict__ PT,
 
 }  // namespace lh
 
+// KV splits of the matrix-core attention: about 256 workgroups, at most one split
+// per block of the longest tile (a 256-token chunk with no prefix runs 4 splits of
+// one block: measured 2.7 us per layer faster than 2 splits of two blocks, the
+// merge included) and the merge's 32. Returns whether k_attn_mfma_long runs.
+// After a long prefix up to twice as many workgroups, two per CU, run there while
+// a split keeps four blocks; a CU's pair takes 7.5 us per block of its splits
+// (k_attn_mfma's one workgroup 5), so it pays where the splits come out half as
+// long, not where a few more workgroups than CUs leave some CUs a second one.
+// Attention and merge, k_attn_mfma and k_attn_mfma_long, in us:
+//   splits half as long: 193 tokens after 2048 positions 49.5, 44.9; 161 after
+//   3072 60.1, 56.4; 65 after 8000 74.8, 64.6; 64 after 10000 62.3, 59.4; 256
+//   after 4000 90.4, 80.8 and after 13000 262, 204;
+//   less than twice the workgroups: 160 after 2048 37.9, 46.5; 128 after 3072
+//   43.4, 50.8; 96 after 4096 44.9, 50.9; 64 after 5000 36.6, 44.8.
+// One tile has 32 splits of either kernel (2, 16 and 32 tokens): after 2048
+// positions 16.8, 18.2, 20.5 and 16.5, 18.9, 20.8; after 4096 22.3, 23.7, 26.4 and
+// 21.1, 23.3, 26.1; after 15872 58.5, 53.2, 54.6 and 54.8, 49.9, 50.9.
+extern "C" int lh_attention_mfma_plan(uint32_t length, uint32_t count, uint32_t* splits)
+{
+    const uint32_t tiles = (count + lh::FA_WG - 1) / lh::FA_WG, units = tiles * LH_KV_HEADS;
+    const uint32_t nb = (length + count + LH_ATTN_BLOCK - 1) / LH_ATTN_BLOCK;
+    auto longest = [&](uint32_t s) { return (nb + s - 1) / s; };   // blocks of a split
+    const uint32_t one = std::max(1u, std::min(256 / units, nb));
+    *splits = one;
+    if (length < lh::FA_LONG_LENGTH) {
+        return 0;
+    }
+    const uint32_t two = std::max(one, std::min({512 / units, nb / 4, 32u}));
+    if (2 * longest(two) > longest(one) + 1 && !(tiles == 1 && length >= lh::FA_LONG_ONE_TILE)) {
+        return 0;
+    }
+    *splits = two;
+    return 1;
+}
+
 extern "C" int lh_launch_attention_mfma(const float* q, const float* kcache_layer,
     const float* vcache_layer, const lh_step_params* params, uint32_t length, uint32_t count,
     uint32_t capacity, float* PM, float* PT, float* PA, float* out, uint16_t* xs, uint32_t xs_tokens,
@@ -1351,23 +1391,9 @@ extern "C" int lh_launch_attention_mfma(const float* q, const float* kcache_laye
         (xs && (xs_tokens < count || !xs_scale))) {
         return -1;
     }
-    // KV splits so that about 256 workgroups run, at most one per block of the
-    // longest tile (a 256-token chunk with no prefix runs 4 splits of one
-    // block: measured 2.7 us per layer faster than 2 splits of two blocks, the
-    // merge included) and the merge's 32. The long variant takes up to twice
-    // as many, two per CU, while a split keeps four blocks.
-    const bool far = length >= lh::FA_LONG_LENGTH;
+    uint32_t splits = 0;
+    const bool far = lh_attention_mfma_plan(length, count, &splits);
     const uint32_t tiles = (count + lh::FA_WG - 1) / lh::FA_WG;
-    const uint32_t nb = (length + count + LH_ATTN_BLOCK - 1) / LH_ATTN_BLOCK;
-    uint32_t splits = 256 / (tiles * LH_KV_HEADS);
-    if (far) {
-        const uint32_t two = 512 / (tiles * LH_KV_HEADS), four = nb / 4;
-        const uint32_t most = two < four ? two : four;
-        splits = splits > most ? splits : most;
-        splits = splits < 32 ? splits : 32;
-    }
-    splits = splits < nb ? splits : nb;
-    splits = splits ? splits : 1;
     const dim3 wgs(tiles * LH_KV_HEADS * splits);
     if (far) {
         hipLaunchKernelGGL(lh::k_attn_mfma_long, wgs, dim3(256), 0, s, q, kcache_layer,

@@ -78,6 +78,8 @@ int lh_launch_attention_mfma(const float *q, const float *kcache_layer, const fl
     const lh_step_params *params, uint32_t length, uint32_t count, uint32_t capacity, float *PM,
     float *PT, float *PA, float *out, uint16_t *xs, uint32_t xs_tokens, float *xs_scale,
     hipStream_t s);
+/* Its KV splits; 1 when the long-prefix kernel runs, 0 otherwise. */
+int lh_attention_mfma_plan(uint32_t length, uint32_t count, uint32_t *splits);
 /* Matrix-core projections of at most 32 tokens (mfma_small.hip); xs: activation
  * planes of `stride` tokens (whole 16-token tiles). qkv: three BF16 planes, RoPE and KV append.
  * o: two FP16 planes scaled per (token, kv head), x += . gateup: two FP16

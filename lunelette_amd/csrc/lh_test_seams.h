@@ -34,6 +34,9 @@ int lunelette_metal_test_set_epoch(struct lunelette_metal *context, uint64_t epo
 /* Whether a decode token at this length runs q|k|v and its attention blocks
  * in one launch on the current device. */
 int lunelette_metal_test_chained(uint32_t length);
+/* The matrix-core attention's KV splits for count tokens after length positions;
+ * 1 when the long-prefix kernel runs, 0 otherwise. */
+int lunelette_metal_test_attention_plan(uint32_t length, uint32_t count, uint32_t *splits);
 /* Overwrites one published host logit. */
 int lunelette_metal_test_set_logit(struct lunelette_metal *context, size_t index, float value);
 /* Arms the allocation counter: the nth device or pinned-host allocation from

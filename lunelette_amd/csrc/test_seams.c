@@ -62,3 +62,8 @@ int lunelette_metal_test_chained(uint32_t length)
 {
     return lh_attention_chained(length);
 }
+
+int lunelette_metal_test_attention_plan(uint32_t length, uint32_t count, uint32_t *splits)
+{
+    return lh_attention_mfma_plan(length, count, splits);
+}

@@ -15,6 +15,7 @@ The reference's own MPS path is pinned only by tolerance (tests/test_metal.m:
   values over 1..69 blocks, ragged token tiles and the causal sentinel of
   tests/test_metal.m:956-999.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -186,6 +187,30 @@ def test_attention_mfma_vs_oracle(gpu, length, count, capacity):
         ref = oracle_lib.attention(REF, q, kpm.reshape(-1), vpm.reshape(-1), 128, 1024,
                                    length, count)
         assert np.max(np.abs(got - ref)) < 2e-4, (length, count)
+
+
+@pytest.mark.parametrize("length,count,capacity,long", [
+    (2047, 16, 4352, 0), (2048, 1, 4352, 0), (2048, 17, 4352, 0), (2048, 33, 4352, 0),
+    (2048, 129, 4352, 0), (2048, 193, 4352, 1), (3000, 211, 4352, 1), (4095, 9, 4352, 0),
+    (4096, 1, 4352, 1), (4097, 16, 4352, 1), (4100, 17, 4352, 1), (4159, 32, 4352, 1),
+    (4200, 33, 4352, 0), (9990, 33, 17920, 1), (9000, 65, 17920, 1)])
+def test_attention_mfma_kernel_choice(gpu, length, count, capacity, long):
+    """Both kernels on both sides of the choice between them, with second
+    16-token subtiles that lie wholly or partly past the last token."""
+    splits = ctypes.c_uint32()
+    assert lh.test_lib().lunelette_metal_test_attention_plan(length, count,
+                                                             ctypes.byref(splits)) == long
+    rng = np.random.default_rng(length + 11 * count)
+    total = length + count
+    q = (rng.normal(size=count * 4096) * 3).astype(np.float32)
+    kpm = rng.normal(size=(total, 1024)).astype(np.float32)
+    vpm = rng.normal(size=(total, 1024)).astype(np.float32)
+    got = gpu_util.attention_on_device(gpu, gpu.lh_attention_mfma, q, kpm, vpm, length, count,
+                                       capacity)
+    mirror = oracle_lib.attention(MIRROR, q, kpm.reshape(-1), vpm.reshape(-1), 128, 1024,
+                                  length, count)
+    assert np.all(np.isfinite(got))
+    assert np.max(np.abs(got - mirror)) < 2e-4, (length, count)
 
 
 def test_attention_mfma_causal_sentinel(gpu):

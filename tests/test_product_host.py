@@ -244,3 +244,40 @@ def test_synthetic_generator_properties(product):
     t = syn.tokens(5, 1, 100000)
     assert t.min() >= 0 and t.max() < 131072 and 68000 < len(np.unique(t)) < 72000
     assert np.array_equal(syn.tokens(5, 1, 10), syn.tokens(5, 1, 10))
+
+
+# Matrix-core attention: (tokens, positions before them) and whether the
+# long-prefix kernel (two four-wave workgroups per CU) is the faster one there.
+ATTENTION_MEASURED = [
+    (256, 2047, 0), (16, 2048, 0), (33, 2048, 0), (160, 2048, 0), (193, 2048, 1), (128, 3072, 0),
+    (161, 3072, 1), (96, 4096, 0), (256, 4096, 1), (7, 4096, 1), (64, 5000, 0), (129, 5000, 1),
+    (64, 8000, 0), (65, 8000, 1), (33, 10000, 1), (64, 15872, 1), (2, 15872, 1)]
+
+
+def attention_plan(length, count):
+    splits = ctypes.c_uint32()
+    return lh.test_lib().lunelette_metal_test_attention_plan(length, count,
+                                                             ctypes.byref(splits)), splits.value
+
+
+@pytest.mark.parametrize("count,length,long", ATTENTION_MEASURED)
+def test_attention_plan_measured_shapes(count, length, long):
+    assert attention_plan(length, count)[0] == long
+
+
+def test_attention_plan_bounds():
+    """Every call of 1 to 256 tokens: at least one split, at most the merge's 32
+    and one per block; past one tile the long-prefix kernel only with splits
+    half as long as those of one workgroup per CU, at least two of them."""
+    for length in list(range(0, 2100, 61)) + [2047, 2048] + list(range(2100, 17664, 509)):
+        for count in range(1, 257):
+            long, splits = attention_plan(length, count)
+            nb, tiles = -(-(length + count) // 64), -(-count // 32)
+            one = max(1, min(256 // (8 * tiles), nb))
+            assert 1 <= splits <= min(32, nb)
+            if not long:
+                assert splits == one
+                continue
+            assert length >= 2048 and splits >= 2 and 8 * tiles * splits <= 512
+            assert nb // splits >= 4 or splits == one
+            assert 2 * -(-nb // splits) <= -(-nb // one) + 1 or (tiles == 1 and length >= 4096)
