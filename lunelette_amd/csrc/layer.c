@@ -239,36 +239,44 @@ static int launched(int status, const char *what)
 
 /* Separate-operator path: every operator is its own kernel, every row dot
  * follows the same canonical schedule as the fused kernels, so results are
- * bitwise identical. */
+ * bitwise identical. Its projections read tensors off a 16-byte boundary by
+ * scalar loads. */
 static int layer_unfused(const lh_layer_weights *w, float *x, float *keys, float *values,
-    lh_workspace *ws, hipStream_t s)
+    lh_workspace *ws, int resident, hipStream_t s)
 {
     const uint32_t n = (uint32_t)ws->count, C = (uint32_t)ws->capacity;
-    const uint8_t *wk = w->qkv + (size_t)LH_QUERY * LH_HIDDEN;
-    const uint8_t *wv = w->qkv + (size_t)(LH_QUERY + LH_KV) * LH_HIDDEN;
+    const int kind = resident ? 2 : 0;
+    const size_t esize = resident ? 4 : 1;
+    const char *wq = resident ? (const char *)w->f32_qkv : (const char *)w->qkv;
+    const char *wk = wq + (size_t)LH_QUERY * LH_HIDDEN * esize;
+    const char *wv = wq + (size_t)(LH_QUERY + LH_KV) * LH_HIDDEN * esize;
+    const void *wo = resident ? (const void *)w->f32_o : (const void *)w->o;
+    const void *wg = resident ? (const void *)w->f32_gate : (const void *)w->gate;
+    const void *wu = resident ? (const void *)w->f32_up : (const void *)w->up;
+    const void *wd = resident ? (const void *)w->f32_down : (const void *)w->down;
     const lh_step_params *params = ws->d_params;
     if (launched(lh_launch_rmsnorm(w->input_norm, x, ws->d_xn, LH_HIDDEN, n, s), "input norm") ||
-        launched(lh_launch_matvec(0, 0, w->qkv, w->scale[0], ws->d_xn, ws->d_qraw, NULL,
+        launched(lh_launch_matvec(kind, 0, wq, w->scale[0], ws->d_xn, ws->d_qraw, NULL,
             LH_QUERY, LH_HIDDEN, n, s), "q") ||
-        launched(lh_launch_matvec(0, 0, wk, w->scale[1], ws->d_xn, ws->d_kraw, NULL,
+        launched(lh_launch_matvec(kind, 0, wk, w->scale[1], ws->d_xn, ws->d_kraw, NULL,
             LH_KV, LH_HIDDEN, n, s), "k") ||
-        launched(lh_launch_matvec(0, 0, wv, w->scale[2], ws->d_xn, ws->d_vraw, NULL,
+        launched(lh_launch_matvec(kind, 0, wv, w->scale[2], ws->d_xn, ws->d_vraw, NULL,
             LH_KV, LH_HIDDEN, n, s), "v") ||
         launched(lh_launch_rope_append(ws->d_qraw, ws->d_kraw, ws->d_vraw, params, n, ws->d_q,
             keys, values, C, s), "rope/append") ||
         launched(lh_launch_attention(ws->d_q, keys, values, ws->d_params, (uint32_t)ws->length, n,
             C, ws->d_PM, ws->d_PT, ws->d_PA, ws->d_arrive, ws->d_bflags, ++ws->epoch,
             ws->handoff_fault, ws->d_attn, s), "attention") ||
-        launched(lh_launch_matvec(0, 0, w->o, w->scale[3], ws->d_attn, x, x, LH_HIDDEN,
+        launched(lh_launch_matvec(kind, 0, wo, w->scale[3], ws->d_attn, x, x, LH_HIDDEN,
             LH_QUERY, n, s), "o") ||
         launched(lh_launch_rmsnorm(w->post_norm, x, ws->d_xn, LH_HIDDEN, n, s), "post norm") ||
-        launched(lh_launch_matvec(0, 0, w->gate, w->scale[4], ws->d_xn, ws->d_gated, NULL,
+        launched(lh_launch_matvec(kind, 0, wg, w->scale[4], ws->d_xn, ws->d_gated, NULL,
             LH_INNER, LH_HIDDEN, n, s), "gate") ||
-        launched(lh_launch_matvec(0, 0, w->up, w->scale[5], ws->d_xn, ws->d_up, NULL,
+        launched(lh_launch_matvec(kind, 0, wu, w->scale[5], ws->d_xn, ws->d_up, NULL,
             LH_INNER, LH_HIDDEN, n, s), "up") ||
         launched(lh_launch_silu_mul(ws->d_gated, ws->d_up, ws->d_gated, (size_t)n * LH_INNER, s),
             "silu") ||
-        launched(lh_launch_matvec(0, 0, w->down, w->scale[6], ws->d_gated, x, x, LH_HIDDEN,
+        launched(lh_launch_matvec(kind, 0, wd, w->scale[6], ws->d_gated, x, x, LH_HIDDEN,
             LH_INNER, n, s), "down")) {
         return -1;
     }
@@ -350,9 +358,11 @@ static int layer_tiles(const lh_layer_weights *w, float *x, float *keys, float *
 #define TILES_MIN 5
 #define TILES_MIN_RESIDENT 2
 
-/* The tiled path loads 16 bytes per lane straight to LDS, which needs 16-byte
- * addresses; tensors elsewhere stay on the row dots. */
-static int tiles_aligned(const lh_layer_weights *w, const float *x, const float *keys,
+/* Whether every tensor of a call lies on a 16-byte boundary. The tiled path
+ * loads 16 bytes per lane straight to LDS, the resident decode kernels as many
+ * to registers; FP8 calls on other tensors stay on the row dots, resident ones
+ * on the separate operators. */
+static int aligned16(const lh_layer_weights *w, const float *x, const float *keys,
     const float *values, int resident)
 {
     const void *p[] = {resident ? (const void *)w->f32_qkv : (const void *)w->qkv,
@@ -408,8 +418,9 @@ int lh_layer_forward(const lh_layer_weights *w, float *d_x, float *d_keys, float
         return -1;
     }
     hipStream_t s = (hipStream_t)stream;
-    const int tiles = ws->count >= (path == LH_PATH_RESIDENT ? TILES_MIN_RESIDENT : TILES_MIN) &&
-        tiles_aligned(w, d_x, d_keys, d_values, path == LH_PATH_RESIDENT);
+    const int aligned = aligned16(w, d_x, d_keys, d_values, path == LH_PATH_RESIDENT);
+    const int tiles = aligned &&
+        ws->count >= (path == LH_PATH_RESIDENT ? TILES_MIN_RESIDENT : TILES_MIN);
     switch (path) {
     case LH_PATH_FUSED:
         return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 0, s)
@@ -418,14 +429,15 @@ int lh_layer_forward(const lh_layer_weights *w, float *d_x, float *d_keys, float
         return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 0, s)
                      : layer_fused(w, d_x, d_keys, d_values, ws, LH_ROWS_FP8_LOOKUP, s);
     case LH_PATH_UNFUSED:
-        return layer_unfused(w, d_x, d_keys, d_values, ws, s);
+        return layer_unfused(w, d_x, d_keys, d_values, ws, 0, s);
     case LH_PATH_RESIDENT:
         if (!w->f32_qkv || !w->f32_o || !w->f32_gate || !w->f32_up || !w->f32_down) {
             lh_set_error("layer_forward: resident path needs FP32 weights");
             return -1;
         }
         return tiles ? layer_tiles(w, d_x, d_keys, d_values, ws, 1, s)
-                     : layer_fused(w, d_x, d_keys, d_values, ws, LH_ROWS_F32, s);
+            : aligned ? layer_fused(w, d_x, d_keys, d_values, ws, LH_ROWS_F32, s)
+                      : layer_unfused(w, d_x, d_keys, d_values, ws, 1, s);
     case LH_PATH_MFMA:
         return lh_layer_forward_mfma(w, d_x, d_keys, d_values, ws, 0, NULL, s);
     default:

@@ -158,6 +158,70 @@ def test_multi_token_layer_unaligned_weights(gpu, layer_host):
         gpu.lh_workspace_destroy(ws)
 
 
+def moved_buffer(a):
+    """The array on the device, 4 bytes past a 16-byte boundary."""
+    raw = np.ascontiguousarray(a).reshape(-1).view(np.uint8)
+    return lh.DeviceBuffer.from_array(np.concatenate([np.zeros(4, np.uint8), raw]))
+
+
+def run_moved_layer(gpu, host, x, kpm, vpm, length, count, capacity, path, moved):
+    """run_layer's output rows and raw caches with the tensors in `moved` off a
+    16-byte boundary."""
+    dev = gpu_util.DeviceLayer(host, resident=path == lh.PATH_RESIDENT)
+    arrays = {"x": x, "keys": gpu_util.keys_to_device(kpm, capacity),
+              "values": gpu_util.kv_to_device_layout(vpm, capacity)}
+    for name in ("input_norm", "post_norm"):
+        arrays[name] = syn.bf16_to_f32(host[name])
+    codes = {"qkv": np.concatenate([host["q"], host["k"], host["v"]], axis=0)}
+    codes.update({n: host[n] for n in ("o", "gate", "up", "down")})
+    dec = gpu_util.decode_table()
+    buffers, at = {}, {}
+    for name in ("x", "keys", "values"):
+        move = name in moved
+        buffers[name] = moved_buffer(arrays[name]) if move else \
+            lh.DeviceBuffer.from_array(arrays[name])
+        at[name] = buffers[name].ptr + (4 if move else 0)
+    for name in set(moved) - set(at):
+        if name in codes:
+            resident = path == lh.PATH_RESIDENT
+            a = dec[codes[name]].astype(np.float32) if resident else codes[name]
+            field = ("f32_" if resident else "") + name
+        else:
+            a, field = arrays[name], name
+        buffers[name] = moved_buffer(a)
+        setattr(dev.weights, field, buffers[name].ptr + 4)
+    ws = gpu.lh_workspace_create(capacity, count)
+    assert ws, lh.last_error()
+    try:
+        ids = np.zeros(count, np.int64)
+        lh.check(gpu.lh_workspace_set_tokens(ws, ids.ctypes.data_as(lh.c_int64_p), length, count,
+                                             None), "set_tokens")
+        lh.check(gpu.lh_layer_forward(dev.weights, at["x"], at["keys"], at["values"], ws, path,
+                                      None), "layer_forward")
+        lh.check(gpu.lh_device_synchronize())
+        return [buffers[n].download(np.uint8)[4 if n in moved else 0:]
+                for n in ("x", "keys", "values")]
+    finally:
+        gpu.lh_workspace_destroy(ws)
+
+
+@pytest.mark.parametrize("count", [1, 9])
+def test_resident_layer_unaligned_tensors(gpu, layer_host, count):
+    """Resident weights, norms and x 4 bytes past a 16-byte boundary: the bits of
+    the aligned call, from the decode kernels' and the tiled path's operators
+    one by one."""
+    length, capacity = 70, 256
+    x = syn.normal_f32(SEED, 9031, count * 3072)
+    kpm = syn.normal_f32(SEED, 9032, length * 1024).reshape(length, 1024)
+    vpm = syn.normal_f32(SEED, 9033, length * 1024).reshape(length, 1024)
+    want, got = (run_moved_layer(gpu, layer_host, x, kpm, vpm, length, count, capacity,
+                                 lh.PATH_RESIDENT, moved)
+                 for moved in ((), ("qkv", "o", "gate", "up", "down", "input_norm", "post_norm",
+                                    "x")))
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
+
+
 @pytest.mark.parametrize("length,count", [(0, 5), (70, 20), (120, 41)])
 def test_multi_token_layer_nonfinite_token(gpu, layer_host, length, count):
     """A token whose input is infinite leaves NaN values in the cache; the
