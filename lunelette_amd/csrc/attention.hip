@@ -44,8 +44,9 @@ namespace lh {
 // workgroups follow the blocks, id 8 * nblk + (4 * (h % 4) + qd) * 8 + h / 4
 // for head h and dimension quarter qd, so each runs on its kv head's XCD and
 // combines from its L2 once the head's blocks have flagged their partials
-// (flags of epoch `cwant`, at most `cspins` polls; see attn_combiner).
-template <AttnTail TAIL>
+// (flags of epoch `cwant`, at most `cspins` polls; see attn_combiner). DIRECT: see
+// attn_block.
+template <AttnTail TAIL, bool DIRECT = true>
 __global__ void __launch_bounds__(256)
 k_attn_blocks(const float* __restrict__ q, const float* __restrict__ kcache,
     const float* __restrict__ vcache, const lh_step_params* __restrict__ params,
@@ -65,8 +66,8 @@ k_attn_blocks(const float* __restrict__ q, const float* __restrict__ kcache,
         return;
     }
     const uint32_t kvh = id & 7, b = (id >> 3) % nblk, t = (id >> 3) / nblk;
-    attn_block<TAIL, false>(q, kcache, vcache, params, capacity, nblk, PM, PT, PA, arrive, nullptr,
-        bflags, epoch, 0, 0, out, b, kvh, t, sh.blocks);
+    attn_block<TAIL, false, DIRECT>(q, kcache, vcache, params, capacity, nblk, PM, PT, PA, arrive,
+        nullptr, bflags, epoch, 0, 0, out, b, kvh, t, sh.blocks);
 }
 
 // grid (32 heads x 4 dimension quarters, count), 256 threads (attn_combine).
@@ -230,7 +231,8 @@ extern "C" int lh_attention_chained(uint32_t length)
 // of at most LH_ATTN_FUSED_BLOCKS combines in its own launch; with bflags
 // set (8 * capacity/64 words; epoch nonzero and new for every launch on them)
 // one token's longer grid runs its blocks and combiners in one launch;
-// otherwise blocks and k_attn_combine run as two launches. fault (test build
+// otherwise blocks and k_attn_combine run as two launches, without direct loads
+// to LDS where q or a cache lies off a 16-byte boundary. fault (test build
 // only): LH_HANDOFF_COMBINERS makes the combiners wait for an epoch no block
 // stores, LH_GIVE_UP_POLLS polls at most, so they give up and write NaN.
 extern "C" int lh_launch_attention(const float* q, const float* kcache_layer,
@@ -243,7 +245,9 @@ extern "C" int lh_launch_attention(const float* q, const float* kcache_layer,
     }
     const uint32_t nblk = lh_attention_blocks(length, count);
     const dim3 grid(LH_KV_HEADS * nblk * count);
-    const bool ok = fused_attention_ok();
+    const bool direct =
+        ((uintptr_t)q | (uintptr_t)kcache_layer | (uintptr_t)vcache_layer) % 16 == 0;
+    const bool ok = direct && fused_attention_ok();
     if (ok && arrive && nblk <= LH_ATTN_FUSED_BLOCKS) {
         hipLaunchKernelGGL(k_attn_blocks<TAIL_COMBINE>, grid, dim3(256), 0, s, q, kcache_layer,
             vcache_layer, params, capacity, nblk, PM, PT, PA, arrive, nullptr, 0ull, 0ull, 0u,
@@ -255,9 +259,9 @@ extern "C" int lh_launch_attention(const float* q, const float* kcache_layer,
             nullptr, bflags, epoch, forced ? epoch + 1 : epoch,
             forced ? LH_GIVE_UP_POLLS : SPIN_LIMIT, out);
     } else {
-        hipLaunchKernelGGL(k_attn_blocks<TAIL_NONE>, grid, dim3(256), 0, s, q, kcache_layer,
-            vcache_layer, params, capacity, nblk, PM, PT, PA, nullptr, nullptr, 0ull, 0ull, 0u,
-            nullptr);
+        hipLaunchKernelGGL((direct ? k_attn_blocks<TAIL_NONE> : k_attn_blocks<TAIL_NONE, false>),
+            grid, dim3(256), 0, s, q, kcache_layer, vcache_layer, params, capacity, nblk, PM, PT,
+            PA, nullptr, nullptr, 0ull, 0ull, 0u, nullptr);
         hipLaunchKernelGGL(k_attn_combine, dim3(LH_HEADS * 4, count), dim3(256), 0, s, PM, PT, PA,
             params, capacity, out);
     }

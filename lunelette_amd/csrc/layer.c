@@ -296,9 +296,10 @@ static int layer_fused(const lh_layer_weights *w, float *x, float *keys, float *
     const void *wg = resident ? (const void *)w->f32_gate : (const void *)w->gate;
     const void *wu = resident ? (const void *)w->f32_up : (const void *)w->up;
     const void *wd = resident ? (const void *)w->f32_down : (const void *)w->down;
-    /* One decode token on FP8 weights: q|k|v and the attention blocks share a
-     * launch. */
-    const int chained = n == 1 && !resident && lh_attention_chained((uint32_t)ws->length);
+    /* One decode token on FP8 weights: q|k|v and the attention blocks, which load
+     * the caches 16 bytes per lane straight to LDS, share a launch. */
+    const int chained = n == 1 && !resident && ((uintptr_t)keys | (uintptr_t)values) % 16 == 0 &&
+        lh_attention_chained((uint32_t)ws->length);
     if ((chained ?
             launched(lh_launch_qkv_attention(lookup, w->qkv, w->scale[0], w->scale[1],
                 w->scale[2], w->input_norm, x, params, (uint32_t)ws->length, ws->d_q, keys,

@@ -346,7 +346,10 @@ __device__ __forceinline__ void attn_block_tail(const float* __restrict__ PM,
 // own XCD, before loading q and patching the current row. A block that gives
 // up writes NaN partials (want differs from the producers' epoch only when
 // the test build forces that path).
-template <AttnTail TAIL, bool CHAINED>
+// DIRECT: q and K go to LDS by direct loads of 16 bytes, which need 16-byte
+// addresses. Otherwise (not CHAINED) they come through registers, whose loads
+// take any float's address; the same words, the same arithmetic.
+template <AttnTail TAIL, bool CHAINED, bool DIRECT = true>
 __device__ __forceinline__ void attn_block(const float* __restrict__ q,
     const float* __restrict__ kcache, const float* __restrict__ vcache,
     const lh_step_params* __restrict__ params, uint32_t capacity, uint32_t nblk,
@@ -370,7 +373,8 @@ __device__ __forceinline__ void attn_block(const float* __restrict__ q,
     // direct loads, then the V tile to registers. Vector loads complete in
     // issue order, so the scores wait for q and K only (an explicit vmcnt(8))
     // and V lands while they run.
-    if (!CHAINED && tid < 128) {
+    static_assert(DIRECT || !CHAINED, "chained blocks load directly");
+    if (DIRECT && !CHAINED && tid < 128) {
         __builtin_amdgcn_global_load_lds(qrow, reinterpret_cast<float4*>(sh.qs) + 64 * wave, 16,
             0, 0);
     }
@@ -379,10 +383,25 @@ __device__ __forceinline__ void attn_block(const float* __restrict__ q,
     // the contiguous 1 KiB of words (8w + i) * 64 .. +63, written to LDS in
     // the same order, so lane l later reads word (8w + i) * 64 + l.
     const uint32_t p = 16 * wave + (lane >> 2), quarter = lane & 3;
+    if constexpr (DIRECT) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        __builtin_amdgcn_global_load_lds(kb + (wave * 8 + i) * 64 + lane,
-            T + (wave * 8 + i) * 64, 16, 0, 0);
+        for (int i = 0; i < 8; i++) {
+            __builtin_amdgcn_global_load_lds(kb + (wave * 8 + i) * 64 + lane,
+                T + (wave * 8 + i) * 64, 16, 0, 0);
+        }
+    } else {
+        auto word = [](const float* src, size_t w) {
+            return make_float4(src[4 * w], src[4 * w + 1], src[4 * w + 2], src[4 * w + 3]);
+        };
+        if (tid < 128) {
+            reinterpret_cast<float4*>(sh.qs)[tid] =
+                word(q + (size_t)t * LH_QUERY + kvh * 4 * LH_HEAD_DIM, tid);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint32_t w = (wave * 8 + i) * 64 + lane;
+            T[w] = word(kcache + tile, w);
+        }
     }
     __builtin_amdgcn_sched_barrier(0);   // V's loads stay behind K's
     // (A native vector type: a float4 struct copy is a memcpy that, with the
@@ -391,7 +410,12 @@ __device__ __forceinline__ void attn_block(const float* __restrict__ q,
     v4f vr[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        vr[i] = reinterpret_cast<const v4f*>(vb)[tid + 256 * i];   // row (tid + 256 i) >> 5
+        if constexpr (DIRECT) {
+            vr[i] = reinterpret_cast<const v4f*>(vb)[tid + 256 * i];   // row (tid + 256 i) >> 5
+        } else {
+            const float* f = vcache + tile + 4 * (tid + 256 * i);
+            vr[i] = v4f{f[0], f[1], f[2], f[3]};
+        }
     }
     // No early exit for blocks past token t's last position (multi-token
     // steps): a branch here lets the compiler sink the V loads below it. Such
@@ -453,6 +477,8 @@ __device__ __forceinline__ void attn_block(const float* __restrict__ q,
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    } else if constexpr (!DIRECT) {
         __syncthreads();
     } else {
         // s_waitcnt vmcnt(8), then a bare barrier: __syncthreads()'s workgroup

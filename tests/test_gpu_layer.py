@@ -205,6 +205,55 @@ def run_moved_layer(gpu, host, x, kpm, vpm, length, count, capacity, path, moved
         gpu.lh_workspace_destroy(ws)
 
 
+@pytest.mark.parametrize("path", [lh.PATH_FUSED, lh.PATH_RESIDENT])
+@pytest.mark.parametrize("length,count", [(70, 1), (70, 9), (1100, 1)])
+def test_layer_unaligned_caches(gpu, layer_host, path, length, count):
+    """Caches 4 bytes past a 16-byte boundary: the bits of the aligned call, also
+    where that shares launches (decode, at most 16 blocks and more)."""
+    capacity = 1280
+    x = syn.normal_f32(SEED, 9041, count * 3072)
+    kpm = syn.normal_f32(SEED, 9042, length * 1024).reshape(length, 1024)
+    vpm = syn.normal_f32(SEED, 9043, length * 1024).reshape(length, 1024)
+    want, got = (run_moved_layer(gpu, layer_host, x, kpm, vpm, length, count, capacity, path,
+                                 moved) for moved in ((), ("keys", "values")))
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
+
+
+@pytest.mark.parametrize("moved", ["q", "keys", "values"])
+@pytest.mark.parametrize("length,count", [(0, 1), (130, 3), (1100, 1), (1030, 2)])
+def test_attention_unaligned_tensors(gpu, length, count, moved):
+    """lh_attention and lh_attention_noalloc with q or a cache 4 bytes past a
+    16-byte boundary, bitwise the mirror."""
+    capacity = 1280
+    rng = np.random.default_rng(length + count)
+    total = length + count
+    q = (rng.normal(size=count * 4096) * 3).astype(np.float32)
+    kpm = rng.normal(size=(total, 1024)).astype(np.float32)
+    vpm = rng.normal(size=(total, 1024)).astype(np.float32)
+    arrays = {"q": q, "keys": gpu_util.keys_to_device(kpm, capacity),
+              "values": gpu_util.kv_to_device_layout(vpm, capacity)}
+    buffers = {n: moved_buffer(a) if n == moved else lh.DeviceBuffer.from_array(a)
+               for n, a in arrays.items()}
+    at = [buffers[n].ptr + (4 if n == moved else 0) for n in ("q", "keys", "values")]
+    want = oracle_lib.attention(MIRROR, q, kpm.reshape(-1), vpm.reshape(-1), 128, 1024, length,
+                                count)
+    ws = gpu.lh_workspace_create(capacity, count)
+    assert ws, lh.last_error()
+    try:
+        ids = np.zeros(count, np.int64)
+        lh.check(gpu.lh_workspace_set_tokens(ws, ids.ctypes.data_as(lh.c_int64_p), length, count,
+                                             None))
+        for entry in ("workspace", "noalloc"):
+            out = lh.DeviceBuffer(count * 4096 * 4)
+            lh.check(gpu.lh_attention(*at, ws, out.ptr, None) if entry == "workspace" else
+                     gpu.lh_attention_noalloc(*at, length, count, capacity, out.ptr, None))
+            lh.check(gpu.lh_device_synchronize())
+            assert np.array_equal(bits(out.download(np.float32)), bits(want)), entry
+    finally:
+        gpu.lh_workspace_destroy(ws)
+
+
 @pytest.mark.parametrize("count", [1, 9])
 def test_resident_layer_unaligned_tensors(gpu, layer_host, count):
     """Resident weights, norms and x 4 bytes past a 16-byte boundary: the bits of

@@ -4,7 +4,9 @@ stand-ins for the launchers that log their names (tests/support/stub_launches.c)
 Tensors off a 16-byte boundary must not reach kernels that load 16 bytes per
 lane without a look at the address: the tiled path and the resident decode
 kernels. Resident calls take the separate operators then, whose projections
-fall back to scalar loads; FP8 calls the row dots.
+fall back to scalar loads; FP8 calls the row dots, a decode token without the
+launch it otherwise shares with its attention blocks, which load the caches that
+way.
 """
 import ctypes
 import os
@@ -86,3 +88,11 @@ def test_unaligned_resident_tensor(stub, moved):
 def test_unaligned_fp8_tensor(stub, moved):
     for count in (4, 9):
         assert route(stub, lh.PATH_FUSED, count, moved) == FP8_ROWS
+
+
+def test_unaligned_cache_is_not_chained(stub):
+    chained = "qkv_attention:%d matvec:0 gateup_silu:%d matvec:0"
+    for path, lookup in ((lh.PATH_FUSED, 0), (lh.PATH_LOOKUP, 1)):
+        assert route(stub, path, 1, chained=1) == chained % (lookup, lookup)
+        for moved in ("keys", "values"):
+            assert route(stub, path, 1, moved, chained=1) == FUSED % (lookup, 0, lookup, 0)
