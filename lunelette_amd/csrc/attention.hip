@@ -379,7 +379,8 @@ extern "C" int lh_launch_embed(const uint16_t* E, const lh_step_params* params, 
 // output goes to xs as the o projection's two FP16 planes (plane stride
 // xs_tokens * 4096, one power of two per (token, kv head) in xs_scale)
 // instead of FP32 rows of out.
-// Measured at 256 tokens after a 4096-token prefix: 88 us (94 us with
+// Measured at 256 tokens after a 4096-token prefix, which k_attn_mfma_long has
+// taken over since: 88 us (94 us with
 // S = Q K^T and P through a per-wave LDS tile, whose reuse of the K planes
 // cost a third barrier per block: per block about 1.5k cycles of barrier
 // skew, 1.5k of staging, 1.0k of the second barrier, 2.1k of QK^T, 1.0k of
@@ -913,7 +914,8 @@ k_attn_mfma(const float* __restrict__ q, const float* __restrict__ kcache,
 // softmax and products overlap the other's, and V is staged behind the softmax,
 // so that both tiles' loads have half a block's time to land (K's during P.V,
 // V's during the scores). Blocks wholly before the tile skip the causal mask,
-// and blocks that raise no maximum the rescaling of O.
+// and blocks that raise no maximum the rescaling of O. Its 33 and more blocks
+// always run in several splits, whose rows k_attn_merge takes.
 // Measured (kernel trace), k_attn_mfma and the former 64-token variant before:
 // 64 tokens after 15872 positions 86 -> 70 us (and 3 us more in the merge of
 // twice as many splits), 256 after 4096 80 -> 77 us (86 us for it at the lower
@@ -936,14 +938,12 @@ __device__ __forceinline__ uint32_t fa_thread()
 __global__ void __launch_bounds__(256, 2)
 k_attn_mfma_long(const float* __restrict__ q, const float* __restrict__ kcache,
     const float* __restrict__ vcache, uint32_t length, uint32_t count, uint32_t capacity,
-    float* __restrict__ PM, float* __restrict__ PT, float* __restrict__ PA, float* __restrict__ out,
-    uint16_t* __restrict__ xs, uint32_t xs_tokens, float* __restrict__ xs_scale)
+    float* __restrict__ PM, float* __restrict__ PT, float* __restrict__ PA)
 {
     constexpr int NP = FA_PASSES;
     __shared__ __attribute__((aligned(16))) uint8_t Kp[2 * FB_KPLANE];
     __shared__ __attribute__((aligned(16))) uint8_t Vp[2 * FB_VPLANE];
     __shared__ float sk[LH_ATTN_BLOCK];
-    __shared__ float gmax[FA_WG][4];
     const FaCoords fc = fa_coords((count + FA_WG - 1) / FA_WG);
     const uint32_t tid = threadIdx.x, lane = tid & 63, kvh = fc.kvh;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1189,72 +1189,26 @@ k_attn_mfma_long(const float* __restrict__ q, const float* __restrict__ kcache,
         load_k(b + 1 < b_end ? b + 1 : b);
         fa_values<NP>(Vp, l16, g, ph, pm, o);
     }
-    // Output planes (one split): each token's four query heads of this kv
-    // head (512 columns, one K split of the o projection) share one power of
-    // two 2^e, their largest magnitude into [2^14, 2^15), before the split
-    // into two FP16 planes; xs_scale[t][kv head] = 2^-e. The heads' maxima
-    // meet in LDS before any wave leaves.
-    if (splits == 1 && xs) {
-#pragma unroll
-        for (int ps = 0; ps < NP; ps++) {
-            float mr = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                mr = fmaxf(mr, fmaxf(fmaxf(fabsf(o[ps][i].x), fabsf(o[ps][i].y)),
-                                     fmaxf(fabsf(o[ps][i].z), fabsf(o[ps][i].w))));
-            }
-            mr = col4_max(mr) / l[ps];
-            if (g == 0) {
-                gmax[FA_TQ * ps + l16][wave] = mr;
-            }
-        }
-        __syncthreads();
-    }
-    // The lane's token and its O^T values: dims 16 i + 4g .. +3.
+    // The lane's token and its O^T values: dims 16 i + 4g .. +3 (the lane again: held
+    // across the block loop it spills).
+    const uint32_t le = fa_thread() & 63, ge = le >> 4;
     const uint32_t nbc = capacity / LH_ATTN_BLOCK;
 #pragma unroll
     for (int ps = 0; ps < NP; ps++) {
-        const uint32_t t = tw + FA_TQ * ps + l16;
+        const uint32_t t = tw + FA_TQ * ps + (le & 15);
         if (t >= count) {
             continue;
         }
-        if (splits == 1) {
-            const float inv = 1.0f / l[ps];
-            if (xs) {
-                const float* gm = gmax[FA_TQ * ps + l16];
-                const int e = row_exponent(fmaxf(fmaxf(gm[0], gm[1]), fmaxf(gm[2], gm[3])));
-                if (g == 0 && wave == 0) {
-                    xs_scale[t * LH_KV_HEADS + kvh] = exp2i(-e);
-                }
-                const float f = exp2i(e);
-                const size_t plane = (size_t)xs_tokens * LH_QUERY;
+        const size_t part = ((size_t)t * LH_HEADS + head) * nbc + z;
+        if (ge == 0) {
+            PM[part] = m[ps];
+            PT[part] = l[ps];
+        }
+        float* dst = PA + part * LH_HEAD_DIM + 4 * ge;
 #pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const fa_floatx4 v = o[ps][i] * (inv * f);
-                    store_f16x2_4(xs, plane,
-                        xs_at(t, head * LH_HEAD_DIM + 16 * i + 4 * g, LH_QUERY),
-                        make_float4(v.x, v.y, v.z, v.w));
-                }
-            } else {
-                float* dst = out + (size_t)t * LH_QUERY + head * LH_HEAD_DIM + 4 * g;
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const fa_floatx4 v = o[ps][i] * inv;
-                    *reinterpret_cast<float4*>(dst + 16 * i) = make_float4(v.x, v.y, v.z, v.w);
-                }
-            }
-        } else {
-            const size_t part = ((size_t)t * LH_HEADS + head) * nbc + z;
-            if (g == 0) {
-                PM[part] = m[ps];
-                PT[part] = l[ps];
-            }
-            float* dst = PA + part * LH_HEAD_DIM + 4 * g;
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                *reinterpret_cast<float4*>(dst + 16 * i) =
-                    make_float4(o[ps][i].x, o[ps][i].y, o[ps][i].z, o[ps][i].w);
-            }
+        for (int i = 0; i < 8; i++) {
+            *reinterpret_cast<float4*>(dst + 16 * i) =
+                make_float4(o[ps][i].x, o[ps][i].y, o[ps][i].z, o[ps][i].w);
         }
     }
 }
@@ -1397,11 +1351,14 @@ extern "C" int lh_launch_attention_mfma(const float* q, const float* kcache_laye
     }
     uint32_t splits = 0;
     const bool far = lh_attention_mfma_plan(length, count, &splits);
+    if (far && splits < 2) {   // k_attn_mfma_long leaves its rows to the merge
+        return -1;
+    }
     const uint32_t tiles = (count + lh::FA_WG - 1) / lh::FA_WG;
     const dim3 wgs(tiles * LH_KV_HEADS * splits);
     if (far) {
         hipLaunchKernelGGL(lh::k_attn_mfma_long, wgs, dim3(256), 0, s, q, kcache_layer,
-            vcache_layer, length, count, capacity, PM, PT, PA, out, xs, xs_tokens, xs_scale);
+            vcache_layer, length, count, capacity, PM, PT, PA);
     } else {
         hipLaunchKernelGGL(lh::k_attn_mfma, wgs, dim3(512), 0, s, q, kcache_layer, vcache_layer,
             length, count, capacity, PM, PT, PA, out, xs, xs_tokens, xs_scale);
