@@ -241,9 +241,8 @@ k_residual_norm_split(const float* __restrict__ partial, size_t split_stride, fl
 // Down-projection input: SiLU(s_g * gate) * (s_u * up) (src/metal_encode.m:
 // 162-171) from the gate|up GEMM partials P[s][m][0..18432) (gate rows first),
 // summed in split order and multiplied by their row scale in_scale[t] (a power
-// of two, exact). groups = 0: S equal K splits; otherwise the stream-K
-// partials of `groups` groups (gemm_stream_tile), S >= every column's
-// segment count. Each of the down projection's DOWN_SPLITS K ranges (576
+// of two, exact): the stream-K partials of `groups` groups (gemm_stream_tile), S >= every
+// column's segment count. Each of the down projection's DOWN_SPLITS K ranges (576
 // columns) gets its own power of two 2^e (its largest magnitude into
 // [2^14, 2^15)) before the split into two FP16 planes; out_scale[t][g] = 2^-e,
 // which the down projection's GEMM applies to that granule's products. grid
@@ -267,8 +266,8 @@ k_split_silu(const float* __restrict__ partial, size_t split_stride, float2 scal
     const float ts = in_scale[t], sg = scales.x, su = scales.y;
     // Segments of the gate column (c4 / 64) and of the up column 36 later.
     constexpr uint32_t STAGES = LH_HIDDEN / BK, UNITS = MAX_N / GN * STAGES;
-    const uint32_t ng = groups ? stream_segments(c4 / 64, STAGES, UNITS, groups) : S;
-    const uint32_t nu = groups ? stream_segments(c4 / 64 + LH_INNER / GN, STAGES, UNITS, groups) : S;
+    const uint32_t ng = stream_segments(c4 / 64, STAGES, UNITS, groups);
+    const uint32_t nu = stream_segments(c4 / 64 + LH_INNER / GN, STAGES, UNITS, groups);
     const float4 g = scale4(sum_segments<S>(row, s4, ng), ts);
     const float4 u = scale4(sum_segments<S>(row + LH_INNER / 4, s4, nu), ts);
     const float4 y = make_float4(silu(g.x * sg) * (u.x * su), silu(g.y * sg) * (u.y * su),
@@ -695,9 +694,9 @@ k_gemm_bf16(const uint8_t* __restrict__ W0, const uint8_t* __restrict__ W1, uint
         nullptr, 0, out);
 }
 
-// 192-row workgroup tiles (48 rows per wave): q|k|v at 4 K splits and o at
-// 8 make 512 workgroups, every two-per-CU slot, where 256-row tiles leave a
-// quarter of them empty.
+// 192-row workgroup tiles (48 rows per wave): at 256 tokens q|k|v at 4 K splits
+// and o and down at 8 make 512 workgroups, every two-per-CU slot, where 256-row
+// tiles leave a quarter of them empty.
 __global__ void __launch_bounds__(256, 2)
 k_gemm_bf16_n3(const uint8_t* __restrict__ W0, const uint8_t* __restrict__ W1, uint32_t boundary,
     uint32_t N, uint32_t K, const uint16_t* __restrict__ xs, uint32_t stride_tokens,
