@@ -103,9 +103,16 @@ enum {
     LH_PATH_FUSED = 0,    /* compact FP8, fused decode-schedule kernels */
     LH_PATH_LOOKUP = 1,   /* same, table decode */
     LH_PATH_UNFUSED = 2,  /* compact FP8, one operator per kernel */
-    LH_PATH_RESIDENT = 3, /* FP32 weights, one operator per kernel */
+    LH_PATH_RESIDENT = 3, /* FP32 weights, fused decode-schedule kernels */
     LH_PATH_MFMA = 4      /* multi-token: MFMA GEMM projections */
 };
+/* FUSED and LOOKUP calls of 5 tokens or more and RESIDENT calls of 2 or more run
+ * their projections and attention on the FP32 matrix instructions in tiles of
+ * 16 tokens, bit for bit the same results; FP8 codes are then decoded by
+ * conversion instructions on either path, LOOKUP's table is not read. This
+ * needs every tensor of the call (weights, norms, d_x, d_keys, d_values) on a
+ * 16-byte boundary: with one elsewhere FUSED and LOOKUP stay on the decode
+ * kernels, one token at a time, and RESIDENT runs one operator per kernel. */
 
 /* KV cache of one layer (capacity a multiple of 64): d_values is
  * [8][capacity][128] FP32 rows; d_keys holds the same [8][capacity][128]

@@ -16,8 +16,13 @@ struct lh_workspace {
     lh_step_params *h_params;      /* pinned */
     lh_step_params *d_params;
     float *d_q, *d_attn;           /* [B][4096] */
-    float *d_gated, *d_up;         /* [B][9216] */
-    float *d_xn;                   /* [B][3072] */
+    /* BT = B, rounded up to whole 16-token tiles where B > 1: the precise
+     * multi-token kernels keep their activations here in tile order
+     * (lh_xt_word) and read whole tiles. There d_xn holds the normalized rows,
+     * d_up the attention's output and d_gated SiLU(gate)*up; elsewhere plain
+     * rows (d_up: the up projection). */
+    float *d_gated, *d_up;         /* [BT][9216] */
+    float *d_xn;                   /* [BT][3072] */
     float *d_qraw, *d_kraw, *d_vraw;
     float *d_PM, *d_PT;            /* [B][32][C/64] block maxima and sums */
     float *d_PA;                   /* [B][32][C/64][128] block P.V partials */

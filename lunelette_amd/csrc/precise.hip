@@ -95,8 +95,11 @@ __device__ __forceinline__ void tile_body(const TileArgs& a)
     constexpr uint32_t NP = 8 * RT;
     constexpr uint32_t RS = 16 * RT + 4;                // reduction row stride: no bank conflicts
     // The 2 NCH stages of a tile take NB buffers in turn, a whole number of
-    // turns per tile, NB - 1 stages of weights ahead; FP32 rows and the
-    // 8-stage projection keep to two, so that two workgroups fit a CU's LDS.
+    // turns per tile, NB - 1 stages of weights ahead. Three turns do not divide
+    // the 8-stage projection. FP32 rows keep to two: with one token tile two
+    // workgroups then fit a CU's LDS (74 KB each, 106 KB with three buffers);
+    // with more tiles one workgroup runs per CU either way, and a third buffer
+    // has not been measured there.
     constexpr int STAGES = 2 * NCH, NB = STAGES % 3 || KIND == K_F32 ? 2 : 3;
     constexpr int UNROLL = 2 * (NB == 3 ? 3 : 1), AHEAD = NB - 1;
     __shared__ u32x4 w0[STAGE_WORDS];
