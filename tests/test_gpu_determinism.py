@@ -6,8 +6,8 @@ stream-K partial is written to its own slot and summed in a fixed order, the
 attention's KV splits merge in split order, and no kernel accumulates with
 atomics. Two contexts (and one context after reset) given the same tokens
 must return the same logit bits and hold the same KV bits, through chunks on
-the 32-token attention kernel (prefixes under 2048) and the 64-token one (from
-2048 on), then through decode steps.
+the attention kernel of short prefixes and, at the chunk after 2048 positions,
+the one of long prefixes, then through decode steps.
 """
 import numpy as np
 import pytest

@@ -94,10 +94,12 @@ def test_mfma_layer_256_after_4096(gpu):
             assert np.max(np.abs(g - w_) / np.max(np.abs(w_), axis=1, keepdims=True)) < 1e-5
 
 
-@pytest.mark.parametrize("length,count", [(3, 5), (40, 100), (7, 130)])
+@pytest.mark.parametrize("length,count", [(3, 5), (3, 33), (21, 50), (60, 64), (40, 100), (7, 130)])
 def test_mfma_layer_small_odd_block(gpu, length, count):
-    """One, two and three 64-token tiles, the last partial (the gate|up
-    stream-K partition takes 36, 30 and 21 groups per XCD there)."""
+    """Past the short-message kernels (5 tokens), one, two and three 64-token
+    tiles: the last one partial or whole, gate|up in a stream-K partition of 36,
+    30 and 21 groups per XCD, q|k|v in 8 K splits for one tile and 4 from two
+    on, down in 16 granule splits up to two tiles and 8 of two granules each."""
     from test_gpu_layer import oracle_layer, run_layer
     host = syn.layer(SEED, 1)
     capacity = 256
@@ -167,11 +169,10 @@ def test_runtime_mps_prefill_then_decode(gpu, prompt):
                                                    (2048, 130, 4352), (3001, 211, 4352),
                                                    (2000, 20, 4352)])
 def test_attention_mfma_vs_oracle(gpu, length, count, capacity):
-    """From a 2048-token prefix and 128 tokens on, the wide kernel runs (64
-    tokens per workgroup); 130 and 211 tokens leave subtiles past the last
-    token, and 2048 + 128 is the smallest such launch. The merge runs with
-    4 (256 tokens), 8 (the wide kernel at 256), 10 and 16 (1000 + 17) and 32
-    (2000 + 20) KV splits."""
+    """Both kernels: the long-prefix one at 4096 + 256 and 3001 + 211; 130 and 211
+    tokens leave a subtile's last rows past the last token. One KV split (3 and
+    5 tokens) and the merge of 4 (0 and 256 + 256), 6 (2048 + 130), 8, 9 (3001 + 211),
+    16 (1000 + 17) and 32 (2000 + 20) of them."""
     rng = np.random.default_rng(length + 7 * count)
     total = length + count
     q = (rng.normal(size=count * 4096) * 3).astype(np.float32)
@@ -189,6 +190,13 @@ def test_attention_mfma_vs_oracle(gpu, length, count, capacity):
         assert np.max(np.abs(got - ref)) < 2e-4, (length, count)
 
 
+def attention_plan(length, count):
+    """Whether the long-prefix kernel runs, and the KV splits."""
+    splits = ctypes.c_uint32()
+    return lh.test_lib().lunelette_metal_test_attention_plan(length, count,
+                                                             ctypes.byref(splits)), splits.value
+
+
 @pytest.mark.parametrize("length,count,capacity,long", [
     (2047, 16, 4352, 0), (2048, 1, 4352, 0), (2048, 17, 4352, 0), (2048, 33, 4352, 0),
     (2048, 129, 4352, 0), (2048, 193, 4352, 1), (3000, 211, 4352, 1), (4095, 9, 4352, 0),
@@ -197,9 +205,7 @@ def test_attention_mfma_vs_oracle(gpu, length, count, capacity):
 def test_attention_mfma_kernel_choice(gpu, length, count, capacity, long):
     """Both kernels on both sides of the choice between them, with second
     16-token subtiles that lie wholly or partly past the last token."""
-    splits = ctypes.c_uint32()
-    assert lh.test_lib().lunelette_metal_test_attention_plan(length, count,
-                                                             ctypes.byref(splits)) == long
+    assert attention_plan(length, count)[0] == long
     rng = np.random.default_rng(length + 11 * count)
     total = length + count
     q = (rng.normal(size=count * 4096) * 3).astype(np.float32)
@@ -234,8 +240,8 @@ def test_mfma_layer_down_input_range(gpu, shift):
     """gate and up scales times 2^shift put SiLU(gate)*up up to about 1e13
     (far past FP16's 65504) or below about 1e-4 (mostly FP16 subnormals):
     the down projection's two FP16 planes carry a power-of-two scale per token
-    and K split, so the layer stays within the matrix-core layer tolerance
-    of the oracle."""
+    and 576-column granule, so the layer stays within the matrix-core layer
+    tolerance of the oracle."""
     from test_gpu_layer import oracle_layer, run_layer
     host = dict(syn.layer(SEED, 2))
     for name in ("scale_gate", "scale_up"):
@@ -253,13 +259,41 @@ def test_mfma_layer_down_input_range(gpu, shift):
     assert np.median(np.abs(gx - wx) / np.maximum(np.abs(wx), 1e-30)) < 1e-5
 
 
+@pytest.mark.parametrize("shift", [14, 0, -14])
+@pytest.mark.parametrize("count", [40, 128, 129, 192])
+def test_mfma_layer_down_granule_scales(gpu, count, shift):
+    """The down projection alone: o's output is 2^-40 of its size, and down's
+    scale times 2^(-2 shift) keeps the MLP the largest part of the layer's output.
+    One, two and three 64-token tiles: one granule per K split up to two, two
+    granules from three on, whose products meet different scales.
+    Tolerance: SiLU(gate)*up and the gate|up input travel as two FP16 planes,
+    each value to 2^-22 of its granule's (row's) largest, and the sums are FP32
+    over up to 9216 terms; 16 * 2^-22 = 4e-6 of a row's largest output (measured
+    9e-7). A granule under another one's power of two would be off by a
+    sixteenth of the output."""
+    from test_gpu_layer import oracle_layer, run_layer
+    host = dict(syn.layer(SEED, 2))
+    for name, e in (("gate", shift), ("up", shift), ("down", -2 * shift), ("o", -40)):
+        host["scale_" + name] = math.ldexp(host["scale_" + name], e)
+    length, capacity = 64, 256
+    x = syn.normal_f32(SEED, 9201, count * 3072)
+    kpm = syn.normal_f32(SEED, 9202, length * 1024).reshape(length, 1024)
+    vpm = syn.normal_f32(SEED, 9203, length * 1024).reshape(length, 1024)
+    got = run_layer(gpu, host, x, kpm, vpm, length, count, capacity, lh.PATH_MFMA)
+    want = oracle_layer(host, x, kpm, vpm, length, count, capacity, MIRROR)
+    gx, wx = got[0].reshape(count, 3072), want[0].reshape(count, 3072)
+    assert np.median(np.abs(wx)) > 1e4   # x is of order 1
+    assert np.max(np.abs(gx - wx) / np.max(np.abs(wx), axis=1, keepdims=True)) < 4e-6
+
+
 def test_mfma_layer_down_granule_gap(gpu):
     """Adjacent 576-column granules of the down input whose largest values
     lie more than 2^100 apart: every gate row of granules 5 and 11 is the code
     -1.0 and the MLP input is positive, so those gates sit near -80 and
     SiLU(gate) * up near 2^-100 there, against about 2^17 in the granules
-    before them. A stream-K segment that crosses such a boundary must not
-    carry its accumulator over by the ratio of the granules' scales (it would
+    before them. At 192 tokens a K split takes two granules, 4 and 5 and 10 and 11
+    among them: each granule's products must meet its own scale before they
+    are added (one accumulator carried over by the ratio of the scales would
     overflow FP32); the layer stays finite and within the matrix-core layer
     tolerance of the oracle."""
     from test_gpu_layer import oracle_layer, run_layer
@@ -320,14 +354,16 @@ def test_attention_ignores_stale_cache_rows(gpu, tail, length, count, capacity):
 
 
 def test_attention_mfma_seeded_shapes(gpu):
-    """Seeded random (prefix, chunk) shapes: both kernels (32-token tiles, and
-    64-token tiles from a 2048-token prefix and 128 tokens on), 1 to 32 KV
-    splits with ragged last splits, ragged token tiles; within 2e-4 of the
-    mirror."""
+    """Seeded random (prefix, chunk) shapes: both kernels, 1 to 32 KV splits with
+    ragged last splits, ragged token tiles; within 2e-4 of the mirror."""
     rng = np.random.default_rng(20251203)
     capacity = 4352
-    for i in range(16):
-        if i % 2:   # the wide kernel's range
+    ran = [0, 0]   # short- and long-prefix kernel
+    for i in range(20):
+        if i >= 16:   # the long-prefix kernel's usual range
+            count = int(rng.integers(193, 257))
+            length = int(rng.integers(2048, capacity - count + 1))
+        elif i % 2:   # around the choice between the kernels
             count = int(rng.integers(128, 161))
             length = int(rng.integers(2048, capacity - count + 1))
         else:
@@ -343,13 +379,15 @@ def test_attention_mfma_seeded_shapes(gpu):
                                       length, count)
         assert np.all(np.isfinite(got)), (length, count)
         assert np.max(np.abs(got - mirror)) < 2e-4, (length, count)
+        ran[attention_plan(length, count)[0]] += 1
+    assert min(ran) >= 4, ran
 
 
 def test_mfma_layer_seeded_shapes(gpu):
     """Seeded random prefixes and chunk sizes through the whole matrix-core
-    layer (ragged 64-token tiles, every stream-K partition of gate|up and
-    down that those counts produce, short and long prefixes), within 1e-3 of
-    each row's largest magnitude of the mirror schedule."""
+    layer (ragged 64-token tiles, every stream-K partition of gate|up and K
+    split of q|k|v and down that those counts produce, short and long prefixes),
+    within 1e-3 of each row's largest magnitude of the mirror schedule."""
     from test_gpu_layer import oracle_layer, run_layer
     host = syn.layer(SEED, 2)
     rng = np.random.default_rng(20251204)
