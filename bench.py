@@ -67,7 +67,7 @@ FP8_WEIGHTS = {"qkv": 6144 * 3072, "o": 3072 * 4096, "gate_up": 2 * 9216 * 3072,
 PREFILL_PLANES = {"qkv": (3, "3 x bf16 (exact split of fp32)"),
                   "o": (2, "2 x fp16 + per-(token, kv head) power-of-two scale (~22 bits)"),
                   "gate_up": (2, "2 x fp16 + per-token power-of-two scale (~22 bits)"),
-                  "down": (2, "2 x fp16 + per-(token, K split) power-of-two scale (~22 bits)")}
+                  "down": (2, "2 x fp16 + per-(token, 576-column granule) power-of-two scale (~22 bits)")}
 # Matrix-core prefill attention: operand formats of its two products.
 PREFILL_ATTENTION = {
     "attention_qk": "Q and K as 2 x fp16 planes (power of two per (token, head) for Q, per "

@@ -34,9 +34,11 @@ struct lh_workspace {
     float *d_yarn;                 /* [C][128]: cos[64], sin[64] per position (decode) */
     float *h_yarn;                 /* host copy of the same rows, filled on first use */
     uint8_t *h_yarn_ready;         /* [C]: row p of h_yarn holds lh_yarn(p) */
-    /* MFMA path: BF16 hi/mid/lo splits of the GEMM inputs, [3][B][K]. */
+    /* MFMA path: activation planes of the GEMM inputs (three BF16 or two FP16
+     * planes in xs_at order, then the FP16 planes' scales) and the GEMMs'
+     * partial sums; B rounded up to 128 tokens. */
     uint16_t *d_split;
-    float *d_gemm;                 /* [B][18432] GEMM outputs */
+    float *d_gemm;
 };
 
 #ifdef __cplusplus
